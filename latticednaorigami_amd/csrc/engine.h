@@ -22,7 +22,7 @@
 // functions (the FourBody walk's parts, the occupancy updates) are inlined
 // into the DEVNI function that calls them, so a binding evaluation runs as
 // a few large functions with its operands in registers.
-#define DEVNI __host__ __device__ __noinline__
+#define DEVNI inline __host__ __device__ __noinline__
 #define DEVIN __host__ __device__ __forceinline__
 
 struct I3 {
@@ -66,45 +66,6 @@ DEV int unit_index(I3 v) {
     return v.z > 0 ? 4 : 5;
 }
 
-// VectorThree::rotate_half (utility.cpp:68-85)
-DEV I3 rotate_half3(I3 v, I3 axis) {
-    int ax = axis.x < 0 ? -axis.x : axis.x;
-    int ay = axis.y < 0 ? -axis.y : axis.y;
-    int az = axis.z < 0 ? -axis.z : axis.z;
-    if (ax == 1 && ay == 0 && az == 0) {
-        return i3(v.x, -v.y, -v.z);
-    }
-    if (ax == 0 && ay == 1 && az == 0) {
-        return i3(-v.x, v.y, -v.z);
-    }
-    if (ax == 0 && ay == 0 && az == 1) {
-        return i3(-v.x, -v.y, v.z);
-    }
-    return v;
-}
-
-// VectorThree::rotate(axis, -1) (utility.cpp:102-142): the quarter turn the
-// ThreeQuarterTurn twist rule uses.
-DEV I3 rotate_minus_quarter3(I3 v, I3 axis) {
-    int dir = -1;
-    int ax = axis.x < 0 ? -axis.x : axis.x;
-    int ay = axis.y < 0 ? -axis.y : axis.y;
-    int az = axis.z < 0 ? -axis.z : axis.z;
-    if (axis.x != ax || axis.y != ay || axis.z != az) {
-        dir = -dir;
-    }
-    if (ax == 1 && ay == 0 && az == 0) {
-        return i3(v.x, -dir * v.z, dir * v.y);
-    }
-    if (ax == 0 && ay == 1 && az == 0) {
-        return i3(-dir * v.z, v.y, dir * v.x);
-    }
-    if (ax == 0 && ay == 0 && az == 1) {
-        return i3(-dir * v.y, dir * v.x, v.z);
-    }
-    return v;
-}
-
 struct Delta {
     double e;
     int st;
@@ -133,8 +94,7 @@ struct Eng {
     int16_t* freel;
     int16_t* tlist;
     int16_t* tcount;
-    uint64_t* hkey;
-    uint32_t* hval;
+    uint32_t* hash;
     int16_t* modified;
     int16_t* assigned;
     PosOre* prev;
@@ -280,8 +240,7 @@ struct Eng {
         freel = (int16_t*)(blk + L.off_free);
         tlist = (int16_t*)(blk + L.off_tlist);
         tcount = (int16_t*)(blk + L.off_tcount);
-        hkey = (uint64_t*)(blk + L.off_hkey);
-        hval = (uint32_t*)(blk + L.off_hval);
+        hash = (uint32_t*)(blk + L.off_hash);
         modified = (int16_t*)(blk + L.off_modified);
         assigned = (int16_t*)(blk + L.off_assigned);
         prev = (PosOre*)(blk + L.off_prev);
@@ -468,27 +427,36 @@ struct Eng {
     DEV int bd(int s) const { return dom[s].bound; }
     DEV bool eb(int s) const { return s >= 0 && dom[s].state == OCC_BOUND; }
     DEV int ident_of(int s) const { return dident[s] + P->ident_lo; }
+    typedef const PosOre* PosList;
+    // a condition every lane computes alike
+    DEV bool agreed(bool b) const { return b; }
+    DEV void rng_begin() { S->rng_idx = 0; }
+    DEV bool all_kinds() const { return true; }
+    DEV void rg_look(const RgCur&) {}
+    DEV int staple_of(int k) const { return ((const int16_t*)sframes)[k]; }
+    // prev[s] = the domain's position and orientation
+    DEV void save_prev(int s) {
+        prev[s].x = dom[s].x;
+        prev[s].y = dom[s].y;
+        prev[s].z = dom[s].z;
+        prev[s].ore = dom[s].ore;
+    }
     DEV double hyb(int a, int b) const { return t_hyb[(size_t)dident[a] * n_ident + dident[b]]; }
     DEV double stk(int a, int b) const { return t_stack[(size_t)dident[a] * n_ident + dident[b]]; }
 
     // ------------------------------------------------------------ site hash
-    DEV uint64_t pkey(I3 p) const {
-        return ((uint64_t)(uint32_t)(p.x + LDO_COORD_OFFSET) << 42) |
-               ((uint64_t)(uint32_t)(p.y + LDO_COORD_OFFSET) << 21) |
-               (uint64_t)(uint32_t)(p.z + LDO_COORD_OFFSET);
-    }
-    DEV int home(uint64_t k) const {
-        return (int)((k * 0x9E3779B97F4A7C15ull) >> (64 - hbits));
-    }
-    DEV int hfind(uint64_t k) const {
-        int i = home(k);
+    // the 16-bit home index of a site (layout.h)
+    DEV int home(I3 p) const { return site_home(p.x, p.y, p.z, hbits); }
+    // index of site p's entry, -1 for an empty site
+    DEV int hfind(I3 p) const {
+        int h = home(p), i = h;
         for (int n = 0; n <= hmask; n++) {
-            uint64_t kk = hkey[i];
-            if (kk == k) {
-                return i;
-            }
-            if (kk == LDO_HASH_EMPTY) {
+            uint32_t v = hash[i];
+            if (v == LDO_HASH_EMPTY) {
                 return -1;
+            }
+            if ((int)(v >> 16) == h && eq3(pos((int)(v & 0xFFFFu)), p)) {
+                return i;
             }
             i = (i + 1) & hmask;
         }
@@ -496,149 +464,65 @@ struct Eng {
     }
     // OrigamiSystem::position_occupancy (origami_system.cpp:193-202)
     DEV int occupancy(I3 p) {
-        int i = hfind(pkey(p));
-        return i < 0 ? OCC_UNASSIGNED : (int)((hval[i] >> 16) & 3u);
+        int i = hfind(p);
+        return i < 0 ? OCC_UNASSIGNED : (int)dom[hash[i] & 0xFFFFu].state;
     }
     DEV int unbound_at(I3 p) {
-        int i = hfind(pkey(p));
-        int s = i < 0 ? -1 : (int)(int16_t)(hval[i] & 0xFFFFu);
+        int i = hfind(p);
+        int s = i < 0 ? -1 : (int)(hash[i] & 0xFFFFu);
         if (s < 0 || s >= nslots) {
             fail(ST_CONSTRAINT);
             return 0;
         }
         return s;
     }
-    DEV void hput(I3 p, int occ, int s) {
+    DEV void check_coord(I3 p) {
         if (p.x <= -LDO_COORD_OFFSET + 2 || p.x >= LDO_COORD_OFFSET - 2 ||
             p.y <= -LDO_COORD_OFFSET + 2 || p.y >= LDO_COORD_OFFSET - 2 ||
             p.z <= -LDO_COORD_OFFSET + 2 || p.z >= LDO_COORD_OFFSET - 2) {
             fail(ST_COORD);
         }
-        uint64_t k = pkey(p);
-        int i = home(k);
-        int n = 0;
-        while (hkey[i] != k && hkey[i] != LDO_HASH_EMPTY) {
-            i = (i + 1) & hmask;
-            if (++n > hmask) {
-                fail(ST_CAPACITY);
+    }
+    // enters domain s as the occupant of site p (in place of the one there)
+    DEV void hput(I3 p, int s) {
+        check_coord(p);
+        int h = home(p), i = h;
+        for (int n = 0; n <= hmask; n++) {
+            uint32_t v = hash[i];
+            if (v == LDO_HASH_EMPTY ||
+                ((int)(v >> 16) == h && ((int)(v & 0xFFFFu) == s || eq3(pos((int)(v & 0xFFFFu)), p)))) {
+                hash[i] = (uint32_t)h << 16 | (uint32_t)s;
                 return;
             }
+            i = (i + 1) & hmask;
         }
-        hkey[i] = k;
-        hval[i] = ((uint32_t)occ << 16) | (uint32_t)(uint16_t)(int16_t)s;
+        fail(ST_CAPACITY);
     }
     // linear-probing deletion with backward shift (Knuth, TAOCP 6.4 Alg. R)
     DEV void herase(I3 p) {
-        int i = hfind(pkey(p));
+        int i = hfind(p);
         if (i < 0) {
             return;
         }
         int j = i;
         for (int n = 0; n <= hmask; n++) {
             j = (j + 1) & hmask;
-            uint64_t kj = hkey[j];
-            if (kj == LDO_HASH_EMPTY) {
+            uint32_t v = hash[j];
+            if (v == LDO_HASH_EMPTY) {
                 break;
             }
-            int k = home(kj);
+            int k = (int)(v >> 16);
             bool stay = (i <= j) ? (i < k && k <= j) : (i < k || k <= j);
             if (stay) {
                 continue;
             }
-            hkey[i] = kj;
-            hval[i] = hval[j];
+            hash[i] = v;
             i = j;
         }
-        hkey[i] = LDO_HASH_EMPTY;
-    }
-
-    // ------------------------------------------------------------ rules
-    // HalfTurnDomain / ThreeQuarterTurnDomain::check_twist_constraint
-    // (domain.cpp:33-40, 69-78)
-    DEV bool twist_ok(int a, I3 ndr, int b) const {
-        I3 r = (dtype == 0) ? rotate_half3(ore(a), ndr)
-                                     : rotate_minus_quarter3(ore(a), ndr);
-        return eq3(r, ore(b));
-    }
-    // check_kink_constraint (domain.cpp:42-57, 80-97)
-    DEV bool kink_ok(int a, I3 ndr, int b) const {
-        I3 oa = ore(a), ob = ore(b);
-        if (eq3(ndr, neg3(oa))) {
-            return false;
-        }
-        if (eq3(ndr, oa)) {
-            if (dtype == 0) {
-                return !eq3(ob, neg3(oa));
-            }
-            return !(eq3(oa, ob) || eq3(oa, neg3(ob)));
-        }
-        if (eq3(ndr, ob) || eq3(ndr, neg3(ob))) {
-            return false;
-        }
-        return true;
-    }
-    // check_junction_constraint (domain.cpp:59-67, 99-118)
-    DEV bool junction_ok(int j1, int j2, int k1, int k2) const {
-        if (dtype == 0) {
-            return true;
-        }
-        I3 nk = sub3(pos(k2), pos(k1));
-        if (eq3(nk, ore(k1))) {
-            I3 n1 = sub3(pos(j2), pos(j1));
-            if (d_of(j1) > d_of(j2)) {
-                n1 = neg3(n1);
-            }
-            if (!twist_ok(k1, n1, k2)) {
-                return false;
-            }
-        }
-        return true;
-    }
-    // doubly_contiguous (origami_potential.cpp:51-68)
-    DEV bool doubly_contig(int a, int b) const {
-        if (cslot_of(a) != cslot_of(b) || d_of(b) != d_of(a) + 1) {
-            return false;
-        }
-        int ba = bd(a), bb = bd(b);
-        if (cslot_of(ba) != cslot_of(bb)) {
-            return false;
-        }
-        int dd = d_of(bb) - d_of(ba);
-        return dd == 1 || dd == -1;
-    }
-    // check_pair_stacked (origami_potential.cpp:70-83)
-    DEV bool pair_stacked(int a, int b) const {
-        if (d_of(a) > d_of(b)) {
-            int t = a;
-            a = b;
-            b = t;
-        }
-        I3 ndr = sub3(pos(b), pos(a));
-        I3 oa = ore(a);
-        if (!eq3(ndr, oa) && !eq3(ndr, neg3(oa))) {
-            return twist_ok(a, ndr, b);
-        }
-        return false;
+        hash[i] = LDO_HASH_EMPTY;
     }
 
     // ------------------------------------------------------------ FourBody
-    DEVIN void fb_single(int h1, int h2, int h3);
-    DEVIN void fb_double(int h1, int h2, int h3);
-    DEVIN void fb_triply(int h1, int h2, int h3);
-    DEVNI void fb_junction(int j1, int j2, int j3, int j4, int k1, int k2);
-    DEVIN void fb_junction_pair(int a, int b, int j);
-    DEVIN void fb_backward_triplets(int a, int b);
-    DEVIN void fb_forward_triplets(int a, int b);
-    DEVIN void fb_central_triplets(int di, int dj);
-    DEVIN void fb_backward_single_junction(int a, int b);
-    DEVIN void fb_backward_outer(int j3, int j4, int k2, int k1);
-    DEVIN void fb_forward_outer(int j1, int j2, int k1, int k2);
-    DEVIN void fb_central_outer(int j1, int j2, int k1, int k2, int k2b);
-    DEVIN void fb_forward_single_junction(int a, int b);
-    DEVIN void fb_central_single_junction(int a, int b);
-    DEVIN void fb_regular_pair(int a, int b, int i);
-    DEVIN void fb_helix_pair(int a, int b, int i, int j);
-    DEVIN void fb_around(int cd, int j);
     DEVNI void fb_terms(int di, int dj);
     DEVIN Delta bind_domain(int di);
 
@@ -658,102 +542,19 @@ struct Eng {
             dom[s].ore = (int8_t)o;
         }
     }
-    DEVNI int add_chain_with(int ident, int uid);
-    DEVNI int add_chain(int ident);
-    DEVNI void delete_chain(int cs);
-    DEVNI void center();
-    DEVNI void set_all_domains();
-    DEVNI void check_all_constraints();
-    DEVNI void update_energy();
-    DEVNI void update_enthalpy_and_entropy();
+#include "engine_decl.h"
 
-    // ------------------------------------------------------------ moves
-    DEVIN int select_random_domain();
-    DEVIN bool test_acceptance(double p);
-    DEVNI bool staple_is_connector(int cs);
-    DEVNI bool scan_for_scaffold(int dom0, int excl_cs);
-    DEVIN int num_bound_staple_domains(int cs);
-    DEVNI void reset_origami();
-    DEVIN double set_growth_point(int gnew, int gold);
-    DEVNI void grow_staple(int cs, int d_i);
-    DEVNI void grow_chain_seq(int cs, int from, int to);
-    DEVNI bool orientation_move();
-    DEVNI bool insert_staple();
-    DEVNI bool delete_staple();
-    DEVIN void cb_unassign_chain(int cs, int from, int to);
-    DEVNI void cb_select_and_set(int d, int prev_d);
-    DEVIN void cb_setup_regrow_old();
-    DEVNI bool cb_test_acceptance();
-    DEVIN void cb_set_old_growth_point(int gnew, int gold);
-    DEVNI bool cb_staple_move();
-    // constraint points
-    DEVNI void cp_reset();
-    DEVIN void cp_add_active(int s, I3 p, int sg);
-    DEVIN void cp_remove_active(int s, bool rec = false);
-    DEVIN void cp_remove_activated(int s);
-    DEVIN void cp_update_endpoints(int s);
-    DEVIN bool cp_endpoint_reached(int s, I3 p);
-    DEVIN bool cp_walks_remain(int s, I3 p);
-    DEVIN bool cp_walks_seg(int s, I3 p, int sg);
-    DEVIN int cp_seg_dir(int cs, int sg);
-    DEVIN bool cp_selected(int b);
-    DEVNI void cp_save_initial();
-    DEVNI void cp_scan_network(int d);
-    DEVNI void cp_find(int first, int count, int dir, int sg);
-    DEVIN bool ct_select_indices(int max_regrowth, int& first, int& count, int& dir);
-    DEVNI void ctcb_grow_chain_scaffold(int first, int count, int dir, bool first_gp = true);
-    DEVNI void ctcb_grow_staple_from(int gold);
-    DEVNI bool ctcb_scaffold_move(int max_regrowth);
-    DEVIN int rg_get_dir(int s);
-    DEVNI double rg_unassign_and_save(bool save);
-    DEVNI double rg_recoil_regrow();
-    DEVNI double rg_set_config(int d, I3 p, int o, int rec);
-    DEVIN void rg_prepare_for_growth(RgCur& c);
-    DEVNI double rg_prepare_for_regrowth(RgCur& c, int rec);
-    DEVNI void rg_restore_endpoints(int d);
-    DEVIN void rg_select(RgCur& c, I3& p, int& o);
-    DEVNI double rg_p_open(const RgCur& c, I3 p, int o);
-    DEVIN bool rg_test_open(double p);
-    DEVNI double rg_calc_weights(const PosOre* actual);
-    DEVNI bool rg_test_avail(RgCur& c);
-    DEVNI void rg_calc_old_c_opens();
-    DEVIN void rg_reset_active(bool remove_first);
-    DEVNI bool rg_regrow_and_accept(bool rm_new, bool rm_opens, bool rm_old);
-    DEVNI bool ctrg_scaffold_move(int max_regrowth);
-    DEVIN void jump_check_stems(int cur, int& tail);
-    DEVNI bool jump_fill(int start, int have, int max_length, int seg_max, int dir, int& tail,
-                         int& last);
-    DEVNI bool jump_select(int max_regrowth);
-    DEVNI bool ctrg_jump_move(int max_regrowth);
-    DEVIN void ctcb_set_first_seg_domain(int stemd);
-    DEVNI void ctcb_jump_grow();
-    DEVNI bool ctcb_jump_move(int max_regrowth);
-    DEVIN bool attempt(int m);
-    DEVNI bool attempt_kind(int kind, int max_regrowth, int m = -1);
-    DEVIN void track_move(int m, bool acc);
-    // learned domain regrowth (lane 0 parts)
-    DEVNI bool chain_connected(int cs);
-    DEVNI int learned_begin(LearnedMove& m);
-    DEVNI void learned_finish(LearnedMove& m);
-    DEVNI int learned_continue(LearnedMove& m);
-    DEVNI int learned_exchange_begin(LearnedMove& m);
-    DEVNI int learned_exchange_continue(LearnedMove& m);
-    DEVNI int learned_path(LearnedMove& m, int i);
-    DEVNI int complement_of(int s);
-    DEVNI int learned_end(LearnedMove& m, bool changed, bool accepted);
-    DEVNI void learned_softmax(const LearnedMove& m, double* w, double& z);
     // channel of the learned proposal's input at site p, leaving domain
     // `excl` out: 0 empty; 1 + o for a scaffold domain, 7 + o for a staple
     // domain only; with two domains of one kind the smaller orientation index
     // (read-only: any lane may call it)
     DEV int site_channel(I3 p, int excl) const {
-        int i = hfind(pkey(p));
+        int i = hfind(p);
         if (i < 0) {
             return 0;
         }
-        int s = (int)(int16_t)(hval[i] & 0xFFFFu);
-        int occ = (int)((hval[i] >> 16) & 3u);
-        int c[2] = {s, (occ != OCC_UNBOUND && s >= 0) ? (int)dom[s].bound : (int)LDO_NONE};
+        int s = (int)(hash[i] & 0xFFFFu);
+        int c[2] = {s, dom[s].state != OCC_UNBOUND ? (int)dom[s].bound : (int)LDO_NONE};
         int scaf = 6, stap = 6;
         for (int k = 0; k < 2; k++) {
             int x = c[k];
@@ -775,25 +576,18 @@ struct Eng {
     }
     // domains at site p other than `excl` (0, 1 or 2)
     DEV int site_count(I3 p, int excl) const {
-        int i = hfind(pkey(p));
+        int i = hfind(p);
         if (i < 0) {
             return 0;
         }
-        int s = (int)(int16_t)(hval[i] & 0xFFFFu);
-        int occ = (int)((hval[i] >> 16) & 3u);
-        int n = (s >= 0 && s != excl) ? 1 : 0;
-        if (occ != OCC_UNBOUND && s >= 0) {
+        int s = (int)(hash[i] & 0xFFFFu);
+        int n = s != excl ? 1 : 0;
+        if (dom[s].state != OCC_UNBOUND) {
             int b = dom[s].bound;
             n += (b >= 0 && b != excl) ? 1 : 0;
         }
         return n;
     }
-    DEVNI void simulate(int64_t steps);
-    DEVNI void begin_interval(int slot, bool recompute);
-    DEVNI int window_op(int staple_offset);
-    DEVNI void count_window_op();
-    DEVNI double calc_move_bias(int staple_offset);
-
     // move-local scratch for the CTCB segment (kept in registers)
     int seg_first, seg_count, seg_dir;
 };

@@ -5,13 +5,18 @@
 // machinery of conserved-topology regrowth (top_constraint_points.cpp).
 // Recursions of the reference (staple-network scans, connector scans,
 // nested staple growth) run on explicit stacks in the replica block.
-#ifndef LDO_ENGINE_MOVES_H
-#define LDO_ENGINE_MOVES_H
-
+//
+// Compiled for Eng, and once more for WEng (engine_wave.h), which defines
+// LDO_WAVE and its own forms of the functions left out then.
 #include "engine.h"
 
+#ifndef LDO_ENG
+#define LDO_ENG Eng
+#endif
+
+#ifndef LDO_WAVE
 // MCMovetype::select_random_domain (movetypes.cpp:98-113)
-DEVIN int Eng::select_random_domain() {
+DEVIN int LDO_ENG::select_random_domain() {
     int idx = uniform_int(0, S->num_domains - 1);
     int n = S->n_chains;
     if (!par) {
@@ -46,17 +51,18 @@ DEVIN int Eng::select_random_domain() {
 }
 
 // MCMovetype::test_acceptance (movetypes.cpp:142-158)
-DEVIN bool Eng::test_acceptance(double p_ratio) {
+DEVIN bool LDO_ENG::test_acceptance(double p_ratio) {
     double p_accept = fmin(1.0, p_ratio) * S->modifier;
     if (p_accept == 1) {
         return true;
     }
     return p_accept > uniform_real();
 }
+#endif // LDO_WAVE
 
 // MCMovetype::scan_for_scaffold_domain (movetypes.cpp:191-232) as an
 // explicit depth-first search; part[] holds the participating chains
-DEVNI bool Eng::scan_for_scaffold(int dom0, int excl_cs) {
+DEVNI bool LDO_ENG::scan_for_scaffold(int dom0, int excl_cs) {
     for (int c = plane(); c < nchain; c += pwidth()) {
         part[c] = 0;
     }
@@ -69,7 +75,7 @@ DEVNI bool Eng::scan_for_scaffold(int dom0, int excl_cs) {
     sp++;
     part[cslot_of(dom0)] = 1;
     while (sp > 0) {
-        NetFrame& f = sframes[sp - 1];
+        auto&& f = sframes[sp - 1];
         int c = cslot_of(f.growth);
         if (f.idx >= ch[c].len) {
             sp--;
@@ -107,7 +113,7 @@ DEVNI bool Eng::scan_for_scaffold(int dom0, int excl_cs) {
 }
 
 // MCMovetype::staple_is_connector (movetypes.cpp:160-177)
-DEVNI bool Eng::staple_is_connector(int cs) {
+DEVNI bool LDO_ENG::staple_is_connector(int cs) {
     for (int d = 0; d < ch[cs].len; d++) {
         int s = slot(cs, d);
         if (dom[s].state != OCC_UNBOUND) {
@@ -124,7 +130,7 @@ DEVNI bool Eng::staple_is_connector(int cs) {
 }
 
 // RegrowthMCMovetype::num_bound_staple_domains (movetypes.cpp:395-405)
-DEVIN int Eng::num_bound_staple_domains(int cs) {
+DEVIN int LDO_ENG::num_bound_staple_domains(int cs) {
     int n = 0;
     for (int d = 0; d < ch[cs].len; d++) {
         int stt = dom[slot(cs, d)].state;
@@ -136,7 +142,7 @@ DEVIN int Eng::num_bound_staple_domains(int cs) {
 }
 
 // MCMovetype::reset_origami (movetypes.cpp:53-86)
-DEVNI void Eng::reset_origami() {
+DEVNI void LDO_ENG::reset_origami() {
     for (int k = 0; k < S->n_assigned; k++) {
         unassign_domain(assigned[k]);
     }
@@ -152,7 +158,7 @@ DEVNI void Eng::reset_origami() {
 }
 
 // RegrowthMCMovetype::set_growth_point (movetypes.cpp:322-341)
-DEVIN double Eng::set_growth_point(int gnew, int gold) {
+DEVIN double LDO_ENG::set_growth_point(int gnew, int gold) {
     double de = set_domain_config(gnew, pos(gold), dom[gold].ore ^ 1);
     if (S->violated) {
         S->rejected = 1;
@@ -164,23 +170,17 @@ DEVIN double Eng::set_growth_point(int gnew, int gold) {
 }
 
 // RegrowthMCMovetype::grow_staple (movetypes.cpp:343-370)
-DEVNI void Eng::grow_staple(int cs, int d_i) {
-    int len = ch[cs].len;
+DEVNI void LDO_ENG::grow_staple(int cs, int d_i) {
     int first = slot(cs, d_i);
-    if (len - d_i > 1) {
-        grow_chain_seq(first, len - d_i, 1);
-    }
-    if (S->rejected) {
-        return;
-    }
-    if (d_i + 1 > 1) {
-        grow_chain_seq(first, d_i + 1, -1);
+#pragma unroll 1
+    for (int way = 0; way < 2 && !S->rejected; way++) {
+        grow_chain_seq(first, way == 0 ? ch[cs].len - d_i : d_i + 1, way == 0 ? 1 : -1);
     }
 }
 
 // grow_chain of the Metropolis (met_movetypes.cpp:50-67) and CB staple
 // (cb_movetypes.cpp:354-361) moves over the domains first, first+dir, ...
-DEVNI void Eng::grow_chain_seq(int first, int count, int dir) {
+DEVNI void LDO_ENG::grow_chain_seq(int first, int count, int dir) {
     int prev_d = first;
     for (int i = 1; i < count; i++) {
         int d = walk(prev_d, dir);
@@ -205,7 +205,7 @@ DEVNI void Eng::grow_chain_seq(int first, int count, int dir) {
 }
 
 // OrientationRotationMCMovetype::internal_attempt_move (orientation_movetype.cpp:30-65)
-DEVNI bool Eng::orientation_move() {
+DEVNI bool LDO_ENG::orientation_move() {
     bool accepted = false;
     int d = select_random_domain();
     if (d < 0) {
@@ -240,7 +240,7 @@ DEVNI bool Eng::orientation_move() {
 
 // MetStapleExchangeMCMovetype::insert_staple + staple_insertion_accepted
 // (met_movetypes.cpp:303-359, 212-253); exchange multipliers are 1
-DEVNI bool Eng::insert_staple() {
+DEVNI bool LDO_ENG::insert_staple() {
     int ntypes = P->L.ntypes;
     int ident = uniform_int(1, ntypes - 1);
     S->trk_type = ident;
@@ -287,7 +287,7 @@ DEVNI bool Eng::insert_staple() {
 
 // MetStapleExchangeMCMovetype::delete_staple + staple_deletion_accepted
 // (met_movetypes.cpp:361-403, 255-301)
-DEVNI bool Eng::delete_staple() {
+DEVNI bool LDO_ENG::delete_staple() {
     int ntypes = P->L.ntypes;
     int ident = uniform_int(1, ntypes - 1);
     S->trk_type = ident;
@@ -304,10 +304,7 @@ DEVNI bool Eng::delete_staple() {
     int len = ch[cs].len;
     for (int d = 0; d < len; d++) {
         int s = slot(cs, d);
-        prev[s].x = dom[s].x;
-        prev[s].y = dom[s].y;
-        prev[s].z = dom[s].z;
-        prev[s].ore = dom[s].ore;
+        save_prev(s);
         push_modified(s);
         S->delta_e += unassign_domain(s);
     }
@@ -327,9 +324,10 @@ DEVNI bool Eng::delete_staple() {
     return accepted;
 }
 
+#ifndef LDO_WAVE
 // CBMCMovetype::calc_biases + calc_bias + select_and_set_config
 // (cb_movetypes.cpp:58-166, 363-387, 486-539)
-DEVNI void Eng::cb_select_and_set(int d, int prev_d) {
+DEVNI void LDO_ENG::cb_select_and_set(int d, int prev_d) {
     I3 pp = pos(prev_d);
     // Per trial site v (the six unit vectors in order): whether it is a
     // candidate, its weight, the orientation it forces (-1: drawn after the
@@ -347,10 +345,10 @@ DEVNI void Eng::cb_select_and_set(int d, int prev_d) {
     bool looked = par && dom[d].state == OCC_UNASSIGNED;
     int occ_l = OCC_UNASSIGNED, ub_l = -1;
     if (looked && plane() < 6) {
-        int hi = hfind(pkey(add3(pp, unit3(plane()))));
+        int hi = hfind(add3(pp, unit3(plane())));
         if (hi >= 0) {
-            occ_l = (int)((hval[hi] >> 16) & 3u);
-            ub_l = (int)(int16_t)(hval[hi] & 0xFFFFu);
+            ub_l = (int)(hash[hi] & 0xFFFFu);
+            occ_l = dom[ub_l].state;
         }
     }
 #pragma unroll
@@ -465,23 +463,21 @@ DEVNI void Eng::cb_select_and_set(int d, int prev_d) {
     }
     push_assigned(d);
 }
+#endif // LDO_WAVE
 
 // CBMCMovetype::unassign_domains (cb_movetypes.cpp:200-213) over the domains
 // of chain cs with d in [from, to)
-DEVIN void Eng::cb_unassign_chain(int cs, int from, int to) {
+DEVIN void LDO_ENG::cb_unassign_chain(int cs, int from, int to) {
     for (int d = from; d < to; d++) {
         int s = slot(cs, d);
-        prev[s].x = dom[s].x;
-        prev[s].y = dom[s].y;
-        prev[s].z = dom[s].z;
-        prev[s].ore = dom[s].ore;
+        save_prev(s);
         push_modified(s);
         unassign_domain(s);
     }
 }
 
 // CBMCMovetype::setup_for_regrow_old (cb_movetypes.cpp:215-225)
-DEVIN void Eng::cb_setup_regrow_old() {
+DEVIN void LDO_ENG::cb_setup_regrow_old() {
     S->regrow_old = 1;
     S->new_bias = S->bias;
     S->new_modifier = S->modifier;
@@ -495,7 +491,7 @@ DEVIN void Eng::cb_setup_regrow_old() {
 }
 
 // CBMCMovetype::test_cb_acceptance (cb_movetypes.cpp:182-198)
-DEVNI bool Eng::cb_test_acceptance() {
+DEVNI bool LDO_ENG::cb_test_acceptance() {
     double ratio = S->new_bias / S->bias;
     if (test_acceptance(ratio)) {
         reset_origami();
@@ -508,14 +504,14 @@ DEVNI bool Eng::cb_test_acceptance() {
 }
 
 // CBMCMovetype::set_old_growth_point (cb_movetypes.cpp:168-180)
-DEVIN void Eng::cb_set_old_growth_point(int gnew, int gold) {
+DEVIN void LDO_ENG::cb_set_old_growth_point(int gnew, int gold) {
     double de = set_checked_domain_config(gnew, pos(gold), old[gnew].ore);
     S->bias *= exp(-de);
     push_assigned(gnew);
 }
 
 // CBStapleRegrowthMCMovetype::internal_attempt_move (cb_movetypes.cpp:292-348)
-DEVNI bool Eng::cb_staple_move() {
+DEVNI bool LDO_ENG::cb_staple_move() {
     if (S->num_staples == 0) {
         S->trk_nost = 1;
         return false;
@@ -530,8 +526,8 @@ DEVNI bool Eng::cb_staple_move() {
     int len = ch[cs].len;
     // (staple domain, partner) pairs of the old configuration, in the
     // replica block: a draw picks one by index
-    int16_t* gnew_l = gpl;
-    int16_t* gold_l = gpl + LDO_MAX_STAPLE_LEN;
+    auto gnew_l = gpl;
+    auto gold_l = gpl + LDO_MAX_STAPLE_LEN;
     int nb = 0;
     for (int d = 0; d < len; d++) {
         int s = slot(cs, d);
@@ -547,24 +543,32 @@ DEVNI bool Eng::cb_staple_move() {
         return false;
     }
     S->bias *= nb;
-    int k = uniform_int(0, nb - 1);
-    cb_unassign_chain(cs, 0, len);
-    double de = set_growth_point(gnew_l[k], gold_l[k]);
-    S->bias *= exp(-de);
-    if (!S->rejected) {
-        grow_staple(cs, d_of(gnew_l[k]));
-    }
-    if (S->rejected) {
-        return false;
-    }
-    S->bias /= num_bound_staple_domains(cs);
-    S->bias *= exp(-calc_move_bias(0)); // add_external_bias (cb_movetypes.cpp:52-56)
-    cb_setup_regrow_old();
-    k = uniform_int(0, nb - 1);
-    cb_unassign_chain(cs, 0, len);
-    cb_set_old_growth_point(gnew_l[k], gold_l[k]);
-    if (!S->rejected) {
-        grow_staple(cs, d_of(gnew_l[k]));
+    // the new configuration, then the old one's weight
+#pragma unroll 1
+    for (int phase = 0; phase < 2; phase++) {
+        if (phase == 1) {
+            cb_setup_regrow_old();
+        }
+        int k = uniform_int(0, nb - 1);
+        int gnew = gnew_l[k], gold = gold_l[k];
+        cb_unassign_chain(cs, 0, len);
+        if (phase == 0) {
+            double de = set_growth_point(gnew, gold);
+            S->bias *= exp(-de);
+        }
+        else {
+            cb_set_old_growth_point(gnew, gold);
+        }
+        if (!S->rejected) {
+            grow_staple(cs, d_of(gnew));
+        }
+        if (phase == 0) {
+            if (S->rejected) {
+                return false;
+            }
+            S->bias /= num_bound_staple_domains(cs);
+            S->bias *= exp(-calc_move_bias(0)); // add_external_bias (cb_movetypes.cpp:52-56)
+        }
     }
     S->modifier = S->new_modifier;
     return cb_test_acceptance();
@@ -572,7 +576,7 @@ DEVNI bool Eng::cb_staple_move() {
 
 // ------------------------------------------------- constraint points
 // Constraintpoints::reset_internal (top_constraint_points.cpp:191-205)
-DEVNI void Eng::cp_reset() {
+DEVNI void LDO_ENG::cp_reset() {
     // -1 in every int8 and int16 entry is the byte pattern 0xff
     fill_section(seg, nslots, 0xffffffffu);
     fill_section(gp, 2 * (int64_t)nslots, 0xffffffffu);
@@ -593,8 +597,9 @@ DEVNI void Eng::cp_reset() {
     n_netds = 0;
 }
 
+#ifndef LDO_WAVE
 // Constraintpoints::add_active_endpoint (:264-278)
-DEVIN void Eng::cp_add_active(int s, I3 p, int sg) {
+DEVIN void LDO_ENG::cp_add_active(int s, I3 p, int sg) {
     if (S->n_active >= P->L.ecap) {
         fail(ST_CAPACITY);
         return;
@@ -611,7 +616,7 @@ DEVIN void Eng::cp_add_active(int s, I3 p, int sg) {
 // Constraintpoints::remove_active_endpoint (:299-320).  With rec, the
 // removed endpoints (get_erased_endpoints) go on top of the erased-endpoint
 // stack as one level.
-DEVIN void Eng::cp_remove_active(int s, bool rec) {
+DEVIN void LDO_ENG::cp_remove_active(int s, bool rec) {
     int sg = seg[s];
     int cs = cslot_of(s), dd = d_of(s);
     int n = S->n_active;
@@ -656,7 +661,7 @@ DEVIN void Eng::cp_remove_active(int s, bool rec) {
 
 // Constraintpoints::remove_activated_endpoint (:322-338): the first active
 // endpoint of the inactive-endpoint domain paired with s
-DEVIN void Eng::cp_remove_activated(int s) {
+DEVIN void LDO_ENG::cp_remove_activated(int s) {
     int e = inact[s];
     if (e < 0) {
         return;
@@ -680,9 +685,10 @@ DEVIN void Eng::cp_remove_activated(int s) {
     }
     S->n_active = n - 1;
 }
+#endif // LDO_WAVE
 
 // Constraintpoints::update_endpoints (:340-349)
-DEVIN void Eng::cp_update_endpoints(int s) {
+DEVIN void LDO_ENG::cp_update_endpoints(int s) {
     cp_remove_active(s);
     int e = inact[s];
     if (e >= 0) {
@@ -690,8 +696,9 @@ DEVIN void Eng::cp_update_endpoints(int s) {
     }
 }
 
+#ifndef LDO_WAVE
 // Constraintpoints::endpoint_reached (:359-372)
-DEVIN bool Eng::cp_endpoint_reached(int s, I3 p) {
+DEVIN bool LDO_ENG::cp_endpoint_reached(int s, I3 p) {
     int sg = seg[s];
     int cs = cslot_of(s), dd = d_of(s);
     int n = S->n_active;
@@ -705,11 +712,12 @@ DEVIN bool Eng::cp_endpoint_reached(int s, I3 p) {
     }
     return pany(hit);
 }
+#endif // LDO_WAVE
 
 // m_domain_to_dir of (chain, segment): the scaffold segments of a
 // non-contiguous selection have their own (0 for an empty one, which the
 // reference never sets)
-DEVIN int Eng::cp_seg_dir(int cs, int sg) {
+DEVIN int LDO_ENG::cp_seg_dir(int cs, int sg) {
     if (cs == 0 && S->n_jsegs > 0) {
         return sdir[sg];
     }
@@ -722,7 +730,7 @@ DEVIN int Eng::cp_seg_dir(int cs, int sg) {
 // (ideal_random_walk.cpp:35-41).  Stem domains look up their segment pair in
 // m_stemd_to_segs, which only holds the scaffold stems of a non-contiguous
 // selection; other stems have no walk constraint.
-DEVIN bool Eng::cp_walks_remain(int s, I3 p) {
+DEVIN bool LDO_ENG::cp_walks_remain(int s, I3 p) {
     if (stem[s] >= 0) {
         if (S->n_jsegs == 0 || cslot_of(s) != 0 || stemseg[s] < 0) {
             return true;
@@ -732,7 +740,8 @@ DEVIN bool Eng::cp_walks_remain(int s, I3 p) {
     return cp_walks_seg(s, p, seg[s]);
 }
 
-DEVIN bool Eng::cp_walks_seg(int s, I3 p, int sg) {
+#ifndef LDO_WAVE
+DEVIN bool LDO_ENG::cp_walks_seg(int s, I3 p, int sg) {
     int cs = cslot_of(s), dd = d_of(s);
     int dir = cp_seg_dir(cs, sg);
     int n = S->n_active;
@@ -769,11 +778,12 @@ DEVIN bool Eng::cp_walks_seg(int s, I3 p, int sg) {
     }
     return !pany(bad);
 }
+#endif // LDO_WAVE
 
 // StapleNetwork::scan_network + scan_staple_topology + make_staple_stack
 // (top_constraint_points.cpp:36-44, 78-170).  The recursion into bound
 // staples runs on frames[]; gps/iaes hold (domain, domain) pairs.
-DEVNI void Eng::cp_scan_network(int d0) {
+DEVNI void LDO_ENG::cp_scan_network(int d0) {
     for (int i = 0; i < n_netds; i++) {
         int s = netds[i];
         netseg[s] = -1;
@@ -806,7 +816,7 @@ DEVNI void Eng::cp_scan_network(int d0) {
         sp++;
     }
     while (sp > 0) {
-        NetFrame& f = frames[sp - 1];
+        auto&& f = frames[sp - 1];
         int ci = cslot_of(f.growth);
         int len = ch[ci].len;
         int gd = d_of(f.growth);
@@ -876,7 +886,7 @@ DEVNI void Eng::cp_scan_network(int d0) {
 }
 
 // whether scaffold domain b is among the selected (m_scaffold_domains)
-DEVIN bool Eng::cp_selected(int b) {
+DEVIN bool LDO_ENG::cp_selected(int b) {
     if (S->n_jsegs > 0) {
         return jdom[b] != 0;
     }
@@ -889,7 +899,7 @@ DEVIN bool Eng::cp_selected(int b) {
 
 // Constraintpoints::find_growthpoints_endpoints (top_constraint_points.cpp:
 // 454-569) for scaffold segment sg: first, first+dir, ... (count domains)
-DEVNI void Eng::cp_find(int first, int count, int dir, int sg) {
+DEVNI void LDO_ENG::cp_find(int first, int count, int dir, int sg) {
     // CTRG grows Constraintpoints::m_d_stack (domains_to_be_regrown): each
     // segment domain, then the domain stack of the network it roots
     bool rec = S->kind == LDO_MOVE_KIND_CTRG || S->kind == LDO_MOVE_KIND_CTRG_JUMP ||
@@ -972,21 +982,50 @@ DEVNI void Eng::cp_find(int first, int count, int dir, int sg) {
     }
 }
 
+#ifndef LDO_WAVE
 // the end of calculate_constraintpoints (top_constraint_points.cpp:220,
 // 247): m_initial_active_endpoints = m_active_endpoints
-DEVNI void Eng::cp_save_initial() {
+DEVNI void LDO_ENG::cp_save_initial() {
     for (int i = plane(), n = S->n_active; i < n; i += pwidth()) {
         active0[i] = active[i];
     }
     S->n_active0 = S->n_active;
 }
 
+// Constraintpoints::reset_active_endpoints (:295-297)
+DEVNI void LDO_ENG::cp_restore_initial() {
+    for (int i = plane(), n = S->n_active0; i < n; i += pwidth()) {
+        active[i] = active0[i];
+    }
+    S->n_active = S->n_active0;
+}
+
+// Staples an internal network takes along, in ascending unique-index order
+// (std::set<int>), listed in the connector-scan frames, which are idle then;
+// returns their number.
+DEVNI int LDO_ENG::ctcb_staples() {
+    int16_t* sl = (int16_t*)sframes;
+    int nst = 0;
+    for (int c2 = 1; c2 < nchain; c2++) {
+        if (regrow[c2] && ch[c2].ident >= 0) {
+            int k = nst++;
+            while (k > 0 && ch[sl[k - 1]].uid > ch[c2].uid) {
+                sl[k] = sl[k - 1];
+                k--;
+            }
+            sl[k] = (int16_t)c2;
+        }
+    }
+    return nst;
+}
+#endif // LDO_WAVE
+
 // CTCBRegrowthMCMovetype::grow_chain (cb_movetypes.cpp:463-484) and
 // grow_staple_and_update_endpoints (:541-562), interleaved through an
 // explicit stack.  Growing starts with the scaffold segment and descends
 // into staples at growthpoints; any rejection unwinds the whole growth.
-DEVNI void Eng::ctcb_grow_chain_scaffold(int first, int count, int dir, bool first_gp) {
-    GrowFrame* stk = gstack;
+DEVNI void LDO_ENG::ctcb_grow_chain_scaffold(int first, int count, int dir, bool first_gp) {
+    auto stk = gstack;
     int sp = 0;
     if (count > 1) {
         GrowFrame f;
@@ -1007,7 +1046,7 @@ DEVNI void Eng::ctcb_grow_chain_scaffold(int first, int count, int dir, bool fir
         stk[sp++] = f;
     }
     while (sp > 0 && !S->rejected && S->status == ST_OK) {
-        GrowFrame& F = stk[sp - 1];
+        auto&& F = stk[sp - 1];
         if (F.kind == 0) {
             if (F.i >= F.count) {
                 sp--;
@@ -1103,7 +1142,7 @@ DEVNI void Eng::ctcb_grow_chain_scaffold(int first, int count, int dir, bool fir
 // CTRegrowthMCMovetype::select_indices (movetypes.cpp:469-510): the
 // segment first, first + dir, ... (count domains), and the active endpoint
 // of the domain past its end
-DEVIN bool Eng::ct_select_indices(int max_regrowth, int& first, int& count, int& dir) {
+DEVIN bool LDO_ENG::ct_select_indices(int max_regrowth, int& first, int& count, int& dir) {
     int guard = 0;
     while (true) {
         int max_len = ns < max_regrowth ? ns : max_regrowth;
@@ -1145,7 +1184,7 @@ DEVIN bool Eng::ct_select_indices(int max_regrowth, int& first, int& count, int&
 }
 
 // CTCBScaffoldRegrowthMCMovetype::internal_attempt_move (cb_movetypes.cpp:680-747)
-DEVNI bool Eng::ctcb_scaffold_move(int max_regrowth) {
+DEVNI bool LDO_ENG::ctcb_scaffold_move(int max_regrowth) {
     S->regrow_old = 0;
     cp_reset();
     int first, count, dir;
@@ -1162,28 +1201,12 @@ DEVNI bool Eng::ctcb_scaffold_move(int max_regrowth) {
     if (!whole_ring) {
         cp_remove_active(first);
     }
-    // staples to be regrown, in ascending unique-index order (std::set<int>);
-    // the list borrows the connector-scan frames, which are idle here
-    int16_t* sl = (int16_t*)sframes;
-    int nst = 0;
-    for (int c2 = 1; c2 < nchain; c2++) {
-        if (regrow[c2] && ch[c2].ident >= 0) {
-            int k = nst++;
-            while (k > 0 && ch[sl[k - 1]].uid > ch[c2].uid) {
-                sl[k] = sl[k - 1];
-                k--;
-            }
-            sl[k] = (int16_t)c2;
-        }
-    }
+    int nst = ctcb_staples();
     S->trk_nst = nst;
     for (int phase = 0; phase < 2; phase++) {
         if (phase == 1) {
             cb_setup_regrow_old();
-            for (int i = plane(), n = S->n_active0; i < n; i += pwidth()) {
-                active[i] = active0[i];
-            }
-            S->n_active = S->n_active0;
+            cp_restore_initial();
             if (!whole_ring) {
                 cp_remove_active(first);
             }
@@ -1191,15 +1214,13 @@ DEVNI bool Eng::ctcb_scaffold_move(int max_regrowth) {
         int d = first;
         for (int i = 1; i < count; i++) {
             d = walk(d, dir);
-            prev[d].x = dom[d].x;
-            prev[d].y = dom[d].y;
-            prev[d].z = dom[d].z;
-            prev[d].ore = dom[d].ore;
+            save_prev(d);
             push_modified(d);
             unassign_domain(d);
         }
         for (int k = 0; k < nst; k++) {
-            cb_unassign_chain(sl[k], 0, ch[sl[k]].len);
+            int cs = staple_of(k);
+            cb_unassign_chain(cs, 0, ch[cs].len);
         }
         ctcb_grow_chain_scaffold(first, count, dir);
         if (phase == 0 && S->rejected) {
@@ -1224,7 +1245,7 @@ DEVNI bool Eng::ctcb_scaffold_move(int max_regrowth) {
 // ascending order are the reference's list after its erasures.
 
 // Constraintpoints::get_dir (top_constraint_points.cpp:179-185)
-DEVIN int Eng::rg_get_dir(int s) {
+DEVIN int LDO_ENG::rg_get_dir(int s) {
     int cs = cslot_of(s);
     int sg = seg[s];
     if (cs == 0 && S->n_jsegs > 0) {
@@ -1237,16 +1258,13 @@ DEVIN int Eng::rg_get_dir(int s) {
 // unassign_domains (:122-129) with neither, and the third pass of the move
 // (whose saved positions are the ones the old configuration keeps in `old`)
 // with modify only
-DEVNI double Eng::rg_unassign_and_save(bool save) {
+DEVNI double LDO_ENG::rg_unassign_and_save(bool save) {
     double de = 0;
     int n = S->n_rgs;
     for (int i = 0; i < n; i++) {
         int d = rgs[i];
         if (save) {
-            prev[d].x = dom[d].x;
-            prev[d].y = dom[d].y;
-            prev[d].z = dom[d].z;
-            prev[d].ore = dom[d].ore;
+            save_prev(d);
         }
         if (i > 0) {
             push_modified(d);
@@ -1265,7 +1283,7 @@ DEVNI double Eng::rg_unassign_and_save(bool save) {
 // records repeat domains the recoil growth recorded first, and their second
 // unassignment in an accepting reset_origami changes nothing but the
 // unassignment count.
-DEVNI double Eng::rg_set_config(int d, I3 p, int o, int rec) {
+DEVNI double LDO_ENG::rg_set_config(int d, I3 p, int o, int rec) {
     double de = set_checked_domain_config(d, p, o);
     if (rec == RG_LIST) {
         push_assigned(d);
@@ -1282,7 +1300,7 @@ DEVNI double Eng::rg_set_config(int d, I3 p, int o, int rec) {
 }
 
 // prepare_for_growth (:243-260)
-DEVIN void Eng::rg_prepare_for_growth(RgCur& c) {
+DEVIN void LDO_ENG::rg_prepare_for_growth(RgCur& c) {
     c.di++;
     c.d = rgs[c.di];
     c.stemd = stem[c.d] >= 0;
@@ -1301,7 +1319,7 @@ DEVIN void Eng::rg_prepare_for_growth(RgCur& c) {
 }
 
 // prepare_for_regrowth (:262-286)
-DEVNI double Eng::rg_prepare_for_regrowth(RgCur& c, int rec) {
+DEVNI double LDO_ENG::rg_prepare_for_regrowth(RgCur& c, int rec) {
     c.di--;
     c.d = rgs[c.di];
     c.dir = rg_get_dir(c.d);
@@ -1330,7 +1348,7 @@ DEVNI double Eng::rg_prepare_for_regrowth(RgCur& c, int rec) {
 }
 
 // restore_endpoints (:288-296)
-DEVNI void Eng::rg_restore_endpoints(int d) {
+DEVNI void LDO_ENG::rg_restore_endpoints(int d) {
     cp_remove_activated(d);
     if (S->er_depth <= 0) {
         fail(ST_MISUSE);
@@ -1339,14 +1357,15 @@ DEVNI void Eng::rg_restore_endpoints(int d) {
     int r = ercnt[--S->er_depth];
     int top = S->er_top - r;
     for (int k = 0; k < r; k++) {
-        const Endpoint& e = erstk[top + k];
+        auto&& e = erstk[top + k];
         cp_add_active(d, i3(e.x, e.y, e.z), seg[d]);
     }
     S->er_top = top;
 }
 
+#ifndef LDO_WAVE
 // select_trial_config (:298-313)
-DEVIN void Eng::rg_select(RgCur& c, I3& p, int& o) {
+DEVIN void LDO_ENG::rg_select(RgCur& c, I3& p, int& o) {
     if (c.stemd) {
         p = pos(c.ref);
         o = dom[c.ref].ore ^ 1;
@@ -1366,7 +1385,7 @@ DEVIN void Eng::rg_select(RgCur& c, I3& p, int& o) {
 }
 
 // calc_p_config_open (:315-343)
-DEVNI double Eng::rg_p_open(const RgCur& c, I3 p, int o) {
+DEVNI double LDO_ENG::rg_p_open(const RgCur& c, I3 p, int o) {
     double de = check_domain_constraints(c.d, p, o);
     if (S->violated) {
         S->violated = 0;
@@ -1387,16 +1406,17 @@ DEVNI double Eng::rg_p_open(const RgCur& c, I3 p, int o) {
 }
 
 // test_config_open (:345-361)
-DEVIN bool Eng::rg_test_open(double p) {
+DEVIN bool LDO_ENG::rg_test_open(double p) {
     p = fmin(1.0, p);
     if (p == 1) {
         return true;
     }
     return p > uniform_real();
 }
+#endif // LDO_WAVE
 
 // recoil_regrow (:177-231)
-DEVNI double Eng::rg_recoil_regrow() {
+DEVNI double LDO_ENG::rg_recoil_regrow() {
     double de = 0;
     int n = S->n_rgs;
     RgCur c;
@@ -1411,6 +1431,7 @@ DEVNI double Eng::rg_recoil_regrow() {
         int o = 0;
         double pc = 0;
         bool open = false;
+        rg_look(c);
         while (!open && c.att != c.maxatt) {
             c.att++;
             rg_select(c, p, o);
@@ -1443,7 +1464,7 @@ DEVNI double Eng::rg_recoil_regrow() {
 }
 
 // test_config_avail (:426-480): feeler growth past level c.di
-DEVNI bool Eng::rg_test_avail(RgCur& c) {
+DEVNI bool LDO_ENG::rg_test_avail(RgCur& c) {
     int n = S->n_rgs;
     int feels = 0;
     if (feels == rg_max_recoils || c.di == n - 1) {
@@ -1455,6 +1476,7 @@ DEVNI bool Eng::rg_test_avail(RgCur& c) {
         I3 p = i3(0, 0, 0);
         int o = 0;
         bool open = false;
+        rg_look(c);
         while (!open && c.att != c.maxatt) {
             c.att++;
             rg_select(c, p, o);
@@ -1497,7 +1519,7 @@ DEVNI bool Eng::rg_test_avail(RgCur& c) {
 // calc_weights (:363-421): the Rosenbluth-like weight of the configuration
 // in `actual`, built level by level from the attempts and configurations
 // the growth left (rgwatt, rgwavail) and the open probabilities (rgopen)
-DEVNI double Eng::rg_calc_weights(const PosOre* actual) {
+DEVNI double LDO_ENG::rg_calc_weights(PosList actual) {
     int n = S->n_rgs;
     double weight = 1;
     RgCur c;
@@ -1517,6 +1539,7 @@ DEVNI double Eng::rg_calc_weights(const PosOre* actual) {
                 att++;
                 I3 p;
                 int o;
+                rg_look(c);
                 rg_select(c, p, o);
                 double pc = rg_p_open(c, p, o);
                 if (rg_test_open(pc)) {
@@ -1533,7 +1556,7 @@ DEVNI double Eng::rg_calc_weights(const PosOre* actual) {
             }
         }
         weight *= avail_cs / rgopen[c.di - 1];
-        const PosOre& a = actual[c.d];
+        auto&& a = actual[c.d];
         rg_set_config(c.d, i3(a.x, a.y, a.z), a.ore, RG_NONE);
     }
     weight /= rgopen[c.di];
@@ -1542,7 +1565,7 @@ DEVNI double Eng::rg_calc_weights(const PosOre* actual) {
 
 // calc_old_c_opens (:482-512): open probabilities of the old configuration
 // (in `old`) and the configurations its growth would have left
-DEVNI void Eng::rg_calc_old_c_opens() {
+DEVNI void LDO_ENG::rg_calc_old_c_opens() {
     int n = S->n_rgs;
     RgCur c;
     c.di = 0;
@@ -1575,11 +1598,8 @@ DEVNI void Eng::rg_calc_old_c_opens() {
 
 // Constraintpoints::reset_active_endpoints (:295-297), then
 // remove_active_endpoint of the segment's first domain when asked
-DEVIN void Eng::rg_reset_active(bool remove_first) {
-    for (int i = plane(), n = S->n_active0; i < n; i += pwidth()) {
-        active[i] = active0[i];
-    }
-    S->n_active = S->n_active0;
+DEVIN void LDO_ENG::rg_reset_active(bool remove_first) {
+    cp_restore_initial();
     if (remove_first) {
         cp_remove_active(rgs[0]);
     }
@@ -1593,7 +1613,7 @@ DEVIN void Eng::rg_reset_active(bool remove_first) {
 // (:152-160).  rm_new, rm_opens and rm_old say whether the stack's first
 // domain loses its active endpoints before the new weights, the old open
 // probabilities and the old weights.
-DEVNI bool Eng::rg_regrow_and_accept(bool rm_new, bool rm_opens, bool rm_old) {
+DEVNI bool LDO_ENG::rg_regrow_and_accept(bool rm_new, bool rm_opens, bool rm_old) {
     int n = S->n_rgs;
     rg_dup = 0;
     S->delta_e += rg_unassign_and_save(true);
@@ -1648,7 +1668,7 @@ DEVNI bool Eng::rg_regrow_and_accept(bool rm_new, bool rm_opens, bool rm_old) {
 
 // CTRGScaffoldRegrowthMCMovetype::internal_attempt_move (:629-689) with
 // setup_constraints (:131-142)
-DEVNI bool Eng::ctrg_scaffold_move(int max_regrowth) {
+DEVNI bool LDO_ENG::ctrg_scaffold_move(int max_regrowth) {
     cp_reset();
     int first, count, dir;
     if (!ct_select_indices(max_regrowth, first, count, dir)) {
@@ -1677,7 +1697,7 @@ DEVNI bool Eng::ctrg_scaffold_move(int max_regrowth) {
 // CTRegrowthMCMovetype::check_for_stemds (movetypes.cpp:704-720): queue the
 // scaffold domains bound to the chain neighbours of the staple domain bound
 // to cur
-DEVIN void Eng::jump_check_stems(int cur, int& tail) {
+DEVIN void LDO_ENG::jump_check_stems(int cur, int& tail) {
     if (dom[cur].state != OCC_BOUND) {
         return;
     }
@@ -1697,7 +1717,7 @@ DEVIN void Eng::jump_check_stems(int cur, int& tail) {
 // CTRegrowthMCMovetype::fill_seg (movetypes.cpp:666-702) for a segment that
 // already holds `have` domains; last is the last domain added (unchanged
 // when none is)
-DEVNI bool Eng::jump_fill(int start, int have, int max_length, int seg_max, int dir, int& tail,
+DEVNI bool LDO_ENG::jump_fill(int start, int have, int max_length, int seg_max, int dir, int& tail,
                           int& last) {
     int cur = start;
     jump_check_stems(cur, tail);
@@ -1729,7 +1749,7 @@ DEVNI bool Eng::jump_fill(int start, int have, int max_length, int seg_max, int 
 // segments (jseg), their directions (sdir), the scaffold stems (jstem) with
 // their growthpoints and segment pairs, and the active endpoints past each
 // segment's end
-DEVNI bool Eng::jump_select(int max_regrowth) {
+DEVNI bool LDO_ENG::jump_select(int max_regrowth) {
     fill_section(jdom, ns, 0u);
     fill_section(stemseg, ns, 0xffffffffu);
     fill_section(sdir, LDO_JUMP_MAX_SEGS, 0u);
@@ -1852,7 +1872,7 @@ DEVNI bool Eng::jump_select(int max_regrowth) {
 }
 
 // CTRGJumpScaffoldRegrowthMCMovetype::internal_attempt_move (:791-853)
-DEVNI bool Eng::ctrg_jump_move(int max_regrowth) {
+DEVNI bool LDO_ENG::ctrg_jump_move(int max_regrowth) {
     cp_reset();
     if (!jump_select(max_regrowth)) {
         return false;
@@ -1880,7 +1900,7 @@ DEVNI bool Eng::ctrg_jump_move(int max_regrowth) {
 // CTCBJumpScaffoldRegrowthMCMovetype::set_first_seg_domain
 // (cb_movetypes.cpp:973-983): a stem binds its growthpoint as in growth
 // from a staple, in the new and the old growth alike
-DEVIN void Eng::ctcb_set_first_seg_domain(int stemd) {
+DEVIN void LDO_ENG::ctcb_set_first_seg_domain(int stemd) {
     int d_old = stem[stemd];
     if (!cp_walks_remain(stemd, pos(d_old))) {
         S->rejected = 1;
@@ -1894,7 +1914,7 @@ DEVIN void Eng::ctcb_set_first_seg_domain(int stemd) {
 // (cb_movetypes.cpp:896-921, 935-960): the first segment with the staple
 // grown from its first domain, then per stem the stem and each of its two
 // segments grown out of it
-DEVNI void Eng::ctcb_jump_grow() {
+DEVNI void LDO_ENG::ctcb_jump_grow() {
     ctcb_grow_chain_scaffold(jseg[0].first, jseg[0].count, jseg[0].dir);
     for (int t = 0; t < S->n_jstems && !S->rejected && S->status == ST_OK; t++) {
         int stemd = jstem[t];
@@ -1910,7 +1930,7 @@ DEVNI void Eng::ctcb_jump_grow() {
 // CTCBJumpScaffoldRegrowthMCMovetype::internal_attempt_move
 // (cb_movetypes.cpp:872-967); unlike the contiguous move, a dead end in the
 // growth of the old configuration rejects too
-DEVNI bool Eng::ctcb_jump_move(int max_regrowth) {
+DEVNI bool LDO_ENG::ctcb_jump_move(int max_regrowth) {
     S->regrow_old = 0;
     cp_reset();
     if (!jump_select(max_regrowth)) {
@@ -1928,31 +1948,19 @@ DEVNI bool Eng::ctcb_jump_move(int max_regrowth) {
     }
     int first = jseg[0].first;
     cp_remove_active(first);
-    int nst = 0;
-    for (int c = 1; c < nchain; c++) {
-        if (regrow[c] && ch[c].ident >= 0) {
-            nst++;
-        }
-    }
-    S->trk_nst = nst;
+    S->trk_nst = ctcb_staples();
     int n = S->n_rgs;
     for (int phase = 0; phase < 2; phase++) {
         if (phase == 1) {
             cb_setup_regrow_old();
-            for (int i = plane(), m = S->n_active0; i < m; i += pwidth()) {
-                active[i] = active0[i];
-            }
-            S->n_active = S->n_active0;
+            cp_restore_initial();
             cp_remove_active(first);
         }
         // CBMCMovetype::unassign_domains (cb_movetypes.cpp:200-213) over the
         // regrowth stack past its first domain
         for (int i = 1; i < n; i++) {
             int d = rgs[i];
-            prev[d].x = dom[d].x;
-            prev[d].y = dom[d].y;
-            prev[d].z = dom[d].z;
-            prev[d].ore = dom[d].ore;
+            save_prev(d);
             push_modified(d);
             unassign_domain(d);
         }
@@ -1970,11 +1978,11 @@ DEVNI bool Eng::ctcb_jump_move(int max_regrowth) {
 
 // MCMovetype::attempt_move and the reset_internal chain (movetypes.cpp:41-51,
 // 242-250; met_movetypes.cpp:45-48, 139-143; cb_movetypes.cpp:44-50, 457-461)
-DEVIN bool Eng::attempt(int m) {
+DEVIN bool LDO_ENG::attempt(int m) {
     return attempt_kind(P->move_kind[m], P->move_maxreg[m], m);
 }
 
-DEVNI bool Eng::attempt_kind(int kind, int max_regrowth, int m) {
+DEVNI bool LDO_ENG::attempt_kind(int kind, int max_regrowth, int m) {
     S->n_modified = 0;
     S->n_assigned = 0;
     S->n_added = 0;
@@ -1992,7 +2000,7 @@ DEVNI bool Eng::attempt_kind(int kind, int max_regrowth, int m) {
         return orientation_move();
     case 1:
         S->kind = LDO_MOVE_KIND_MET;
-        S->trk_ins = uniform_real() < 0.5 ? 1 : 0;
+        S->trk_ins = agreed(uniform_real() < 0.5) ? 1 : 0;
         return S->trk_ins ? insert_staple() : delete_staple();
     case 2:
         S->kind = LDO_MOVE_KIND_CB;
@@ -2001,17 +2009,26 @@ DEVNI bool Eng::attempt_kind(int kind, int max_regrowth, int m) {
         S->kind = LDO_MOVE_KIND_CTCB;
         return ctcb_scaffold_move(max_regrowth);
     case 4:
+        if (!all_kinds()) {
+            break;
+        }
         S->kind = LDO_MOVE_KIND_CTRG;
         rg_max_recoils = m >= 0 ? P->move_recoils[m] : 0;
         rg_max_att = m >= 0 ? P->move_cattempts[m] : 36;
         return ctrg_scaffold_move(max_regrowth);
     case 5:
+        if (!all_kinds()) {
+            break;
+        }
         S->kind = LDO_MOVE_KIND_CTRG_JUMP;
         rg_max_recoils = m >= 0 ? P->move_recoils[m] : 0;
         rg_max_att = m >= 0 ? P->move_cattempts[m] : 36;
         rg_max_segreg = m >= 0 ? P->move_segreg[m] : 0;
         return ctrg_jump_move(max_regrowth);
     case 6:
+        if (!all_kinds()) {
+            break;
+        }
         // a CTCB move throughout (grow_chain, calc_bias), on a jump selection
         S->kind = LDO_MOVE_KIND_CTCB;
         rg_max_segreg = m >= 0 ? P->move_segreg[m] : 0;
@@ -2021,13 +2038,14 @@ DEVNI bool Eng::attempt_kind(int kind, int max_regrowth, int m) {
     return false;
 }
 
+#ifndef LDO_WAVE
 // MCMovetype::add_tracker (movetypes.cpp:41-51) for the move kinds whose
 // summaries list tracked counts: MetStapleExchange by staple type and
 // direction (met_movetypes.cpp:145-190), CBStapleRegrowth by staple type
 // unless there were no staples (cb_movetypes.cpp:264-290),
 // CTCBScaffoldRegrowth by segment length and staples regrown
 // (cb_movetypes.cpp:626-678)
-DEVIN void Eng::track_move(int m, bool acc) {
+DEVIN void LDO_ENG::track_move(int m, bool acc) {
     S->last_move = m;
     S->last_acc = acc ? 1 : 0;
     int T = P->L.ntypes;
@@ -2071,13 +2089,13 @@ DEVIN void Eng::track_move(int m, bool acc) {
 
 // GCMCSimulation::simulate (simulation.cpp:568-653) and select_movetype
 // (:655-665); output writers are host-side and not part of the step
-DEVNI void Eng::simulate(int64_t steps) {
+DEVNI void LDO_ENG::simulate(int64_t steps) {
     for (int64_t n = 0; n < steps; n++) {
         if (S->status != ST_OK) {
             break;
         }
         S->step += 1;
-        S->rng_idx = 0;
+        rng_begin();
         double prob = uniform_real();
         int m = 0;
         while (m < P->n_moves && !(prob < P->move_cum[m])) {
@@ -2109,11 +2127,12 @@ DEVNI void Eng::simulate(int64_t steps) {
 // USGCMCSimulation::update_internal (us_simulation.cpp:262-266): one visit
 // of the window's order parameter after each step.  A slot belongs to one
 // replica for a whole sweep, so its bins have a single writer.
-DEVNI void Eng::count_window_op() {
+DEVNI void LDO_ENG::count_window_op() {
     int p = window_op(0);
     int b = (p >= 0 && p < P->grid_len) ? p : P->grid_len;
     P->hist[(size_t)S->temp_slot * (P->grid_len + 1) + b] += 1;
 }
+#endif // LDO_WAVE
 
 // update_control_qs of the PT drivers (ptmc_simulation.cpp:595-680): switch
 // to the tables of ladder slot `slot` and, with `recompute` (update_temp),
@@ -2123,7 +2142,7 @@ DEVNI void Eng::count_window_op() {
 // 1057-1063); on later visits of the key the initiation terms keep their
 // last values.  slot_key numbers the keys.  Without `recompute` (a window
 // swap at one temperature) only the tables are selected.
-DEVNI void Eng::begin_interval(int slot_, bool recompute) {
+DEVNI void LDO_ENG::begin_interval(int slot_, bool recompute) {
     S->temp_slot = slot_;
     if (recompute) {
         uint64_t bit = 1ull << (P->slot_key != nullptr ? P->slot_key[slot_] : slot_);
@@ -2138,9 +2157,10 @@ DEVNI void Eng::begin_interval(int slot_, bool recompute) {
     }
 }
 
+#ifndef LDO_WAVE
 // the window's order parameter: fully bound pairs (numfulldomains) or
 // staples (numstaples), the latter offset while a deletion is tested
-DEVNI int Eng::window_op(int staple_offset) {
+DEVNI int LDO_ENG::window_op(int staple_offset) {
     const ldo_window& w = P->windows[S->temp_slot];
     if (w.op == LDO_OP_NUMSTAPLES) {
         return S->num_staples + staple_offset;
@@ -2152,7 +2172,7 @@ DEVNI int Eng::window_op(int staple_offset) {
 // (order_params.cpp:595-603; bias_functions.cpp:484-496) for the replica's
 // umbrella window: a LinearStepWell restraint (bias_functions.cpp:139-151)
 // then a Grid bias (242-284).  The stored values belong to the window.
-DEVNI double Eng::calc_move_bias(int staple_offset) {
+DEVNI double LDO_ENG::calc_move_bias(int staple_offset) {
     if (P->windows == nullptr) {
         return 0;
     }
@@ -2178,6 +2198,7 @@ DEVNI double Eng::calc_move_bias(int staple_offset) {
     st[1] = g;
     return diff * w.bias_mult;
 }
+#endif // LDO_WAVE
 
 // ------------------------------------------------------ learned proposal
 // Learned domain regrowth (no reference counterpart): a staple end domain d
@@ -2189,7 +2210,7 @@ DEVNI double Eng::calc_move_bias(int staple_offset) {
 // regrowth instead.  Returns 1 when the lanes must build the context and
 // evaluate the network, 0 when the attempt is complete.
 // whether staple chain cs reaches the scaffold through bound pairs
-DEVNI bool Eng::chain_connected(int cs) {
+DEVNI bool LDO_ENG::chain_connected(int cs) {
     for (int k = 0; k < ch[cs].len; k++) {
         int b = dom[slot(cs, k)].bound;
         if (b < 0 || cslot_of(b) == cs) {
@@ -2202,10 +2223,10 @@ DEVNI bool Eng::chain_connected(int cs) {
     return false;
 }
 
-DEVNI int Eng::learned_begin(LearnedMove& m) {
+DEVNI int LDO_ENG::learned_begin(LearnedMove& m) {
     S->rng_sub = 1;
     S->learned_step += 1;
-    S->rng_idx = 0;
+    rng_begin();
     m.mode = 0;
     int ls = P->learned_slot;
     if (uniform_real() < P->learned_fallback) {
@@ -2256,7 +2277,7 @@ DEVNI int Eng::learned_begin(LearnedMove& m) {
 }
 
 // unnormalised masked softmax of the network's logits and its sum
-DEVNI void Eng::learned_softmax(const LearnedMove& m, double* w, double& z) {
+DEVNI void LDO_ENG::learned_softmax(const LearnedMove& m, double* w, double& z) {
     float mx = -INFINITY;
     for (int k = 0; k < 36; k++) {
         if (m.legal[k / 6]) {
@@ -2270,7 +2291,7 @@ DEVNI void Eng::learned_softmax(const LearnedMove& m, double* w, double& z) {
     }
 }
 
-DEVNI int Eng::learned_continue(LearnedMove& m) {
+DEVNI int LDO_ENG::learned_continue(LearnedMove& m) {
     if (m.kind == 1) {
         learned_finish(m);
         return 0;
@@ -2278,7 +2299,7 @@ DEVNI int Eng::learned_continue(LearnedMove& m) {
     return learned_exchange_continue(m);
 }
 
-DEVNI void Eng::learned_finish(LearnedMove& m) {
+DEVNI void LDO_ENG::learned_finish(LearnedMove& m) {
     int ls = P->learned_slot;
     double w[36];
     double z;
@@ -2316,10 +2337,7 @@ DEVNI void Eng::learned_finish(LearnedMove& m) {
         int d = m.d;
         int cs = cslot_of(d);
         int partner = dom[d].bound;
-        prev[d].x = dom[d].x;
-        prev[d].y = dom[d].y;
-        prev[d].z = dom[d].z;
-        prev[d].ore = dom[d].ore;
+        save_prev(d);
         push_modified(d);
         double de = unassign_domain(d);
         I3 pn = add3(i3(m.ax, m.ay, m.az), unit3(kn / 6));
@@ -2359,7 +2377,7 @@ DEVNI void Eng::learned_finish(LearnedMove& m) {
 // insertion and its inverse for a deletion (N counted with the staple).
 // the scaffold domain a staple domain grows onto: scaffold domain v - 1 for
 // identity v when it carries identity -v, else none
-DEVNI int Eng::complement_of(int s) {
+DEVNI int LDO_ENG::complement_of(int s) {
     int v = ident_of(s);
     if (v < 1 || v > ns) {
         return -1;
@@ -2368,7 +2386,7 @@ DEVNI int Eng::complement_of(int s) {
     return ident_of(x) == -v ? x : -1;
 }
 
-DEVNI int Eng::learned_end(LearnedMove& m, bool changed, bool accepted) {
+DEVNI int LDO_ENG::learned_end(LearnedMove& m, bool changed, bool accepted) {
     if (changed && !accepted) {
         reset_origami();
         calc_move_bias(0);
@@ -2381,7 +2399,7 @@ DEVNI int Eng::learned_end(LearnedMove& m, bool changed, bool accepted) {
 
 // sets up the scoring of growth path i of staple m.cs (domain i grows, the
 // other is placed by the network) for a deletion
-DEVNI int Eng::learned_path(LearnedMove& m, int i) {
+DEVNI int LDO_ENG::learned_path(LearnedMove& m, int i) {
     int gi = slot(m.cs, i), dj = slot(m.cs, 1 - i);
     int idv = ident_of(dj);
     m.a = gi;
@@ -2397,7 +2415,7 @@ DEVNI int Eng::learned_path(LearnedMove& m, int i) {
     return 1;
 }
 
-DEVNI int Eng::learned_exchange_begin(LearnedMove& m) {
+DEVNI int LDO_ENG::learned_exchange_begin(LearnedMove& m) {
     S->n_modified = 0;
     S->n_assigned = 0;
     S->n_added = 0;
@@ -2467,7 +2485,7 @@ DEVNI int Eng::learned_exchange_begin(LearnedMove& m) {
     return learned_path(m, m.valid[0] ? 0 : 1);
 }
 
-DEVNI int Eng::learned_exchange_continue(LearnedMove& m) {
+DEVNI int LDO_ENG::learned_exchange_continue(LearnedMove& m) {
     double w[36];
     double z;
     learned_softmax(m, w, z);
@@ -2532,10 +2550,7 @@ DEVNI int Eng::learned_exchange_continue(LearnedMove& m) {
     double n_before = (double)S->num_staples;
     for (int k = 0; k < 2; k++) {
         int s = slot(cs, k);
-        prev[s].x = dom[s].x;
-        prev[s].y = dom[s].y;
-        prev[s].z = dom[s].z;
-        prev[s].ore = dom[s].ore;
+        save_prev(s);
         push_modified(s);
         S->delta_e += unassign_domain(s);
     }
@@ -2548,5 +2563,3 @@ DEVNI int Eng::learned_exchange_continue(LearnedMove& m) {
     }
     return learned_end(m, true, acc);
 }
-
-#endif

@@ -4,13 +4,19 @@
 // site hash, domain set/unset with FP64 energy accumulation in the
 // reference's order, chain add/delete with the working chain order, and the
 // periodic centring / full constraint check / energy recomputation.
-#ifndef LDO_ENGINE_SYSTEM_H
-#define LDO_ENGINE_SYSTEM_H
-
+//
+// Compiled for Eng, and once more for WEng (engine_wave.h), which defines
+// LDO_WAVE and its own domain operations and chain lists.
 #include "engine.h"
 
+#ifndef LDO_ENG
+#define LDO_ENG Eng
+#endif
+
+#ifndef LDO_WAVE
+
 // OrigamiSystem::update_occupancies (origami_system.cpp:770-806)
-DEVIN void Eng::update_occupancies(int s, I3 p) {
+DEVIN void LDO_ENG::update_occupancies(int s, I3 p) {
     int occ = occupancy(p);
     if (occ == OCC_UNBOUND) {
         int dj = unbound_at(p);
@@ -28,7 +34,7 @@ DEVIN void Eng::update_occupancies(int s, I3 p) {
         }
         // a bound site keeps the domain placed last (the learned proposal
         // reads both domains of a site through it)
-        hput(p, nst, s);
+        hput(p, s);
         dom[s].state = (int8_t)nst;
         dom[dj].state = (int8_t)nst;
         dom[dj].bound = (int16_t)s;
@@ -36,7 +42,7 @@ DEVIN void Eng::update_occupancies(int s, I3 p) {
     }
     else if (occ == OCC_UNASSIGNED) {
         dom[s].state = OCC_UNBOUND;
-        hput(p, OCC_UNBOUND, s);
+        hput(p, s);
     }
     else {
         fail(ST_CONSTRAINT);
@@ -44,7 +50,7 @@ DEVIN void Eng::update_occupancies(int s, I3 p) {
 }
 
 // OrigamiSystem::internal_check_domain_constraints (:828-871)
-DEVIN Delta Eng::internal_check(int s, I3 p, int o) {
+DEVIN Delta LDO_ENG::internal_check(int s, I3 p, int o) {
     Delta dc;
     dc.e = 0;
     dc.st = 0;
@@ -76,7 +82,7 @@ DEVIN Delta Eng::internal_check(int s, I3 p, int o) {
 // OrigamiSystem::internal_unassign_domain (:695-760).  need_delta=false is
 // used where the caller discards the returned change (a peek, or undoing a
 // violating placement); the stacking walk is then skipped.
-DEVIN Delta Eng::internal_unassign(int s, bool need_delta) {
+DEVIN Delta LDO_ENG::internal_unassign(int s, bool need_delta) {
     Delta dc;
     dc.e = 0;
     dc.st = 0;
@@ -107,7 +113,7 @@ DEVIN Delta Eng::internal_unassign(int s, bool need_delta) {
         dom[s].bound = LDO_NONE;
         dom[dj].bound = LDO_NONE;
         dom[s].state = OCC_UNASSIGNED;
-        hput(pos(s), OCC_UNBOUND, dj);
+        hput(pos(s), dj);
         dom[dj].state = OCC_UNBOUND;
         dc.e += de;
     }
@@ -123,7 +129,7 @@ DEVIN Delta Eng::internal_unassign(int s, bool need_delta) {
 }
 
 // OrigamiSystem::check_domain_constraints (:343-355)
-DEVNI double Eng::check_domain_constraints(int s, I3 p, int o) {
+DEVNI double LDO_ENG::check_domain_constraints(int s, I3 p, int o) {
     // An unassigned domain checked at an empty site: placing it and taking it
     // off again leaves the site hash as it was (the key is appended at the
     // end of its probe run, so its removal shifts nothing back) and the
@@ -143,7 +149,7 @@ DEVNI double Eng::check_domain_constraints(int s, I3 p, int o) {
 }
 
 // OrigamiSystem::unassign_domain (:375-385)
-DEVNI double Eng::unassign_domain(int s) {
+DEVNI double LDO_ENG::unassign_domain(int s) {
     Delta dc = internal_unassign(s, true);
     S->energy += dc.e;
     S->num_stacked += dc.st;
@@ -153,7 +159,7 @@ DEVNI double Eng::unassign_domain(int s) {
 }
 
 // OrigamiSystem::set_checked_domain_config (:478-515)
-DEVNI double Eng::set_checked_domain_config(int s, I3 p, int o) {
+DEVNI double LDO_ENG::set_checked_domain_config(int s, I3 p, int o) {
     dom[s].x = p.x;
     dom[s].y = p.y;
     dom[s].z = p.z;
@@ -181,7 +187,7 @@ DEVNI double Eng::set_checked_domain_config(int s, I3 p, int o) {
 }
 
 // OrigamiSystem::set_domain_config (:517-541)
-DEVNI double Eng::set_domain_config(int s, I3 p, int o) {
+DEVNI double LDO_ENG::set_domain_config(int s, I3 p, int o) {
     if (dom[s].state != OCC_UNASSIGNED) {
         fail(ST_CONSTRAINT);
         return 0;
@@ -200,7 +206,7 @@ DEVNI double Eng::set_domain_config(int s, I3 p, int o) {
 }
 
 // OrigamiSystem::add_chain(ident, index) (:402-443)
-DEVNI int Eng::add_chain_with(int ident, int uid) {
+DEVNI int LDO_ENG::add_chain_with(int ident, int uid) {
     int cs;
     if (ident == 0) {
         cs = 0;
@@ -240,15 +246,18 @@ DEVNI int Eng::add_chain_with(int ident, int uid) {
     return cs;
 }
 
+#endif // LDO_WAVE
+
 // OrigamiSystem::add_chain(ident) (:387-400)
-DEVNI int Eng::add_chain(int ident) {
+DEVNI int LDO_ENG::add_chain(int ident) {
     S->current_c_i += 1;
     S->energy += init_e;
     return add_chain_with(ident, S->current_c_i);
 }
 
+#ifndef LDO_WAVE
 // OrigamiSystem::delete_chain (:445-472)
-DEVNI void Eng::delete_chain(int cs) {
+DEVNI void LDO_ENG::delete_chain(int cs) {
     int w = 0;
     while (w < S->n_chains && order[w] != cs) {
         w++;
@@ -276,13 +285,13 @@ DEVNI void Eng::delete_chain(int cs) {
     S->energy -= init_e;
 }
 
+#endif // LDO_WAVE
+
 // OrigamiSystem::center (:553-571): translate so that the centring scaffold
 // domain sits at the origin and rebuild the site hash
-DEVNI void Eng::center() {
+DEVNI void LDO_ENG::center() {
     I3 ref = pos(slot(0, P->centering_domain));
-    for (int i = 0; i < P->L.hcap; i++) {
-        hkey[i] = LDO_HASH_EMPTY;
-    }
+    fill_section(hash, 4 * (int64_t)P->L.hcap, LDO_HASH_EMPTY);
     for (int w = 0; w < S->n_chains; w++) {
         int cs = order[w];
         for (int d = 0; d < ch[cs].len; d++) {
@@ -291,19 +300,15 @@ DEVNI void Eng::center() {
             dom[s].x = np.x;
             dom[s].y = np.y;
             dom[s].z = np.z;
-            int stt = dom[s].state;
-            if (stt == OCC_UNBOUND) {
-                hput(np, OCC_UNBOUND, s);
-            }
-            else if (stt != OCC_UNASSIGNED) {
-                hput(np, stt, s);
+            if (dom[s].state != OCC_UNASSIGNED) {
+                hput(np, s);
             }
         }
     }
 }
 
 // OrigamiSystem::set_all_domains() + check_distance_constraints (:573-586, 357-373)
-DEVNI void Eng::set_all_domains() {
+DEVNI void LDO_ENG::set_all_domains() {
     for (int w = 0; w < S->n_chains; w++) {
         int cs = order[w];
         for (int d = 0; d < ch[cs].len; d++) {
@@ -335,7 +340,7 @@ DEVNI void Eng::set_all_domains() {
 }
 
 // OrigamiSystem::check_all_constraints (:267-325)
-DEVNI void Eng::check_all_constraints() {
+DEVNI void LDO_ENG::check_all_constraints() {
     if (S->num_unassigned != 0) {
         fail(ST_CONSTRAINT);
         return;
@@ -358,7 +363,7 @@ DEVNI void Eng::check_all_constraints() {
         return;
     }
     double eps = 0.000001;
-    if (S->energy < -eps || S->energy > eps) {
+    if (agreed(S->energy < -eps || S->energy > eps)) {
         set_all_domains();
         fail(ST_CONSTRAINT);
         return;
@@ -369,7 +374,7 @@ DEVNI void Eng::check_all_constraints() {
 }
 
 // OrigamiSystem::update_energy (:808-826)
-DEVNI void Eng::update_energy() {
+DEVNI void LDO_ENG::update_energy() {
     for (int w = 0; w < S->n_chains; w++) {
         int cs = order[w];
         for (int d = 0; d < ch[cs].len; d++) {
@@ -383,13 +388,11 @@ DEVNI void Eng::update_energy() {
 
 // OrigamiSystem::update_enthalpy_and_entropy (:204-246); the per-slot flags
 // stand in for the reference's std::set of accounted partners
-DEVNI void Eng::update_enthalpy_and_entropy() {
+DEVNI void LDO_ENG::update_enthalpy_and_entropy() {
     size_t n2 = (size_t)P->n_ident * P->n_ident;
     const double* th = P->hyb_h + (size_t)S->temp_slot * n2;
     const double* ts = P->hyb_s + (size_t)S->temp_slot * n2;
-    for (int s = 0; s < nslots; s++) {
-        netds_flag[s] = 0;
-    }
+    fill_section(netds_flag, nslots, 0u);
     double h = 0, e = 0;
     for (int w = 0; w < S->n_chains; w++) {
         int cs = order[w];
@@ -413,5 +416,3 @@ DEVNI void Eng::update_enthalpy_and_entropy() {
     S->hyb_s = e;
     S->stack_e = S->energy - (h - e);
 }
-
-#endif

@@ -8,22 +8,36 @@
 //
 // Domains live in fixed slots: slots [0, ns) are the scaffold, staple chain
 // slot k (1 <= k <= max_total_staples) owns slots ns + (k-1)*lmax .. + lmax.
-// A lattice site is one entry of an open-addressed, linear-probing hash
-// keyed by the packed position; its value holds the occupancy state and, for
-// an unbound site, the slot of the domain on it.
+// An occupied lattice site is one 4-byte entry of an open-addressed,
+// linear-probing hash: the site's home index and the slot of the domain placed
+// on it last, whose record holds the site's position and occupancy state.
 #ifndef LDO_LAYOUT_H
 #define LDO_LAYOUT_H
 
 #include <stdint.h>
 
+#if defined(__HIP__)
+#define LDO_HD __attribute__((host)) __attribute__((device)) inline __attribute__((always_inline))
+#else
+#define LDO_HD inline
+#endif
+
 #include "../../include/ldo.h"
 
 #define LDO_NONE ((int16_t)-1)
-#define LDO_HASH_EMPTY 0xFFFFFFFFFFFFFFFFull
-#define LDO_COORD_BITS 21
+#define LDO_HASH_EMPTY 0xFFFFFFFFu // no slot is 0xFFFF
 #define LDO_COORD_OFFSET (1 << 20)
 
 enum { OCC_UNASSIGNED = 0, OCC_UNBOUND = 1, OCC_BOUND = 2, OCC_MISBOUND = 3 };
+
+// Home index of a site in a hash of 2^bits entries (bits <= 16): the high bits
+// of a multiplicative hash of the three coordinates (odd 32-bit constants:
+// the golden ratio's and its multiples by 3 and 7).
+LDO_HD int site_home(int x, int y, int z, int bits) {
+    uint32_t h = (uint32_t)x * 0x9E3779B9u + (uint32_t)y * 0xDAA66D2Bu + (uint32_t)z * 0x5384540Fu;
+    h ^= h >> 15;
+    return (int)((h * 0x9E3779B1u) >> (32 - bits));
+}
 
 // Domain record, 16 bytes.
 struct DomRec {
@@ -45,7 +59,7 @@ struct ChainRec {
     int16_t len;
 };
 
-// Active endpoint of the constraint-point machinery, 16 bytes.
+// Active endpoint of the constraint-point machinery, 20 bytes.
 struct Endpoint {
     int16_t cslot; // chain slot of the endpoint domain's chain
     int16_t d;     // domain index within the chain (scaffolds up to 30000 domains)
@@ -170,7 +184,7 @@ struct Layout {
     int32_t ecap;      // endpoint list capacity
     int32_t track_len; // per-move tracking counters (see off_track)
     int64_t off_dom, off_dident, off_chain, off_order, off_free, off_tlist, off_tcount;
-    int64_t off_hkey, off_hval, off_modified, off_assigned, off_prev, off_old;
+    int64_t off_hash, off_modified, off_assigned, off_prev, off_old;
     int64_t off_seg, off_gp, off_stem, off_inact, off_netseg, off_netds_flag;
     int64_t off_checked, off_netcs, off_regrow, off_dir0, off_dir1;
     int64_t off_active, off_active0, off_gps, off_iaes, off_netds, off_frames;
@@ -192,6 +206,9 @@ struct Layout {
     // length attempts[ns+1], accepts[ns+1]; CTRG jump attempts, accepts;
     // CTCB jump by staples regrown attempts[smax+1], accepts[smax+1]
     int64_t off_track;
+    // the sections up to here are what a sweep keeps in LDS; the endpoint
+    // lists and the tracking counters follow
+    int64_t stage;
     int64_t bytes; // block size (multiple of 256)
 };
 
@@ -225,6 +242,7 @@ struct Params {
     const int32_t* type_len;   // [ntypes]
     const int16_t* type_ident; // [ntypes * type_ident_stride] table index of each domain
     int32_t type_ident_stride;
+    int32_t stack_one;         // every pair has the same stacking energy
     const double* hyb_e;       // [n_slots * n_ident^2]
     const double* hyb_h;
     const double* hyb_s;

@@ -75,8 +75,7 @@ Layout make_layout(int ns, int lmax, int smax, int ntypes, int tcap, bool rg, bo
     take(L.off_free, C * 2);
     take(L.off_tlist, (int64_t)ntypes * tcap * 2);
     take(L.off_tcount, (int64_t)ntypes * 2);
-    take(L.off_hkey, (int64_t)hcap * 8);
-    take(L.off_hval, (int64_t)hcap * 4);
+    take(L.off_hash, (int64_t)hcap * 4);
     take(L.off_modified, 2 * S * 2);
     take(L.off_assigned, 2 * S * 2);
     take(L.off_prev, S * (int64_t)sizeof(PosOre));
@@ -92,8 +91,6 @@ Layout make_layout(int ns, int lmax, int smax, int ntypes, int tcap, bool rg, bo
     take(L.off_regrow, C);
     take(L.off_dir0, C);
     take(L.off_dir1, C);
-    take(L.off_active, (int64_t)L.ecap * (int64_t)sizeof(Endpoint));
-    take(L.off_active0, (int64_t)L.ecap * (int64_t)sizeof(Endpoint));
     take(L.off_gps, 2 * S * 2);
     take(L.off_iaes, 2 * S * 2);
     take(L.off_netds, S * 2);
@@ -122,6 +119,9 @@ Layout make_layout(int ns, int lmax, int smax, int ntypes, int tcap, bool rg, bo
     take(L.off_jstem, J * LDO_JUMP_MAX_SEGS);
     take(L.off_stemseg, J * ns);
     take(L.off_sdir, J * LDO_JUMP_MAX_SEGS);
+    L.stage = off;
+    take(L.off_active, (int64_t)L.ecap * (int64_t)sizeof(Endpoint));
+    take(L.off_active0, (int64_t)L.ecap * (int64_t)sizeof(Endpoint));
     L.track_len = 6 * ntypes + 4 * (ns + 1) + 4 * (smax + 1) + 2;
     take(L.off_track, (int64_t)L.track_len * 8);
     L.bytes = round_up(off, 256);
@@ -313,6 +313,7 @@ void make_plan(const ldo_system_desc* sys, const ldo_run_params* run, int32_t n_
         }
     }
     P.type_ident_stride = stride;
+    P.stack_one = sys->stacking_pot != LDO_STACK_SEQUENCESPECIFIC;
     // ladder and per-replica chemical potentials (molarity_to_chempots,
     // chempots_to_reduced_chempots: origami_system.cpp:965-989)
     int nst = sys->n_chain_types - 1;

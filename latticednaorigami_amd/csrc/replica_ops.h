@@ -9,10 +9,17 @@
 #define LDO_REPLICA_OPS_H
 
 #include "engine.h"
-#include "engine_fourbody.h"
-#include "engine_moves.h"
-#include "engine_system.h"
+#include "engine_wave.h"
 #include "layout.h"
+
+// whether the moveset holds a recoil-growth or jump move
+LDO_HD bool wave_all_kinds(const Params& P) {
+    bool a = false;
+    for (int m = 0; m < P.n_moves; m++) {
+        a = a || P.move_kind[m] > LDO_MOVE_KIND_CTCB;
+    }
+    return a;
+}
 
 // Build (mode 0: OrigamiSystem constructor) or replace (mode 1: set_config)
 // replica r's configuration.  c_idx/c_ident hold n_chains unique indices and
@@ -30,7 +37,7 @@ DEV void init_replica(const Params& P, int r, const int32_t* c_idx, const int32_
         S->status = ST_OK;
         e.attach(&P, blk, r);
         for (int i = 0; i < P.L.hcap; i++) {
-            e.hkey[i] = LDO_HASH_EMPTY;
+            e.hash[i] = LDO_HASH_EMPTY;
         }
         for (int c = 0; c < P.L.nchain; c++) {
             e.ch[c].ident = -1;
@@ -111,6 +118,30 @@ DEV void sweep_replica_on(Eng& e, const Params& P, int r, char* blk, int64_t ste
     if (rep_slot != nullptr) {
         e.update_enthalpy_and_entropy();
     }
+}
+
+// The same with the wavefront engine, on a copy of the block's staged part in
+// `lds` (wave_lds_bytes).  ALL: the moveset holds a recoil-growth or jump move.
+template <bool ALL>
+DEV void sweep_wave(const Params& P, int r, char* blk, lds_t lds, int64_t steps,
+                    const int32_t* rep_slot) {
+    WEng e;
+    e.kinds = ALL;
+    e.attach(&P, blk, lds, r);
+    if (e.sc.status != ST_OK) {
+        return;
+    }
+    if (rep_slot != nullptr) {
+        int slot = uni(rep_slot[r]);
+        bool moved = P.slot_key != nullptr &&
+                     uni(P.slot_key[slot]) != uni(P.slot_key[e.sc.temp_slot]);
+        e.begin_interval(slot, P.exchange_mode != LDO_EXCHANGE_WINDOWS || moved);
+    }
+    e.simulate(steps);
+    if (rep_slot != nullptr) {
+        e.update_enthalpy_and_entropy();
+    }
+    e.store_scalars();
 }
 
 DEV void sweep_replica(const Params& P, int r, int64_t steps, const int32_t* rep_slot,

@@ -37,6 +37,7 @@
 #include "layout.h"
 #include "plan.h"
 #include "replica_ops.h"
+#include "sweep_wave.h"
 
 // ------------------------------------------------------------------ kernels
 __device__ __forceinline__ int replica_of_thread(const Params& P, bool& active) {
@@ -64,18 +65,6 @@ extern "C" __global__ void ldo_init_kernel(Params P, const int32_t* c_idx, const
     init_replica(P, r, c_idx, c_ident, c_pos, c_ore, n_chains, mode, rep_slot);
 }
 
-// The replica a workgroup of the one-replica-per-workgroup sweeps runs.
-// Workgroups are dealt to the 8 XCDs round-robin, so workgroup b runs on XCD
-// b % 8; when the ladder divides into 8 equal runs of slots, XCD x takes the
-// replicas of slots [x R/8, (x+1) R/8), so that each XCD's L2 holds the
-// energy tables of few temperatures (slots are temperature-major).  q_to_rep
-// (slot -> replica) is the exchange's permutation, or null for the identity.
-__device__ inline int replica_of_block(const Params& P, const int32_t* q_to_rep) {
-    int b = blockIdx.x, R = P.n_replicas;
-    int q = (R % 8 == 0) ? (b % 8) * (R / 8) + b / 8 : b;
-    return q_to_rep != nullptr ? q_to_rep[q] : q;
-}
-
 // With a wavefront per replica, its 64 lanes run the replica's chain
 // together (lane-parallel sections spread independent reads over them); the
 // engine object sits in LDS, so its section pointers are not re-read from
@@ -94,37 +83,6 @@ extern "C" __global__ void ldo_sweep_kernel(Params P, int64_t steps, const int32
     if ((int)blockIdx.x < P.n_replicas) {
         int r = replica_of_block(P, q_to_rep);
         sweep_replica_on(lds_engine, P, r, P.blocks + (size_t)r * P.L.bytes, steps, rep_slot, 1);
-    }
-}
-
-// One workgroup of 64 lanes per replica.  Every access of the Markov chain
-// to its replica state (the block, the engine's section pointers and the
-// launch parameters) goes to LDS instead of device memory or scratch.  The
-// dynamic LDS holds the block (P.L.bytes, a multiple of 256); the host picks
-// this kernel only when that fits.
-extern "C" __global__ void __launch_bounds__(64)
-    ldo_sweep_lds_kernel(Params P, int64_t steps, const int32_t* rep_slot,
-                         const int32_t* q_to_rep) {
-    extern __shared__ uint4 lds_block[];
-    __shared__ Params lds_params;
-    __shared__ Eng lds_engine;
-    if ((int)blockIdx.x >= P.n_replicas) {
-        return;
-    }
-    int r = replica_of_block(P, q_to_rep);
-    size_t n16 = (size_t)P.L.bytes / 16;
-    uint4* g = (uint4*)(P.blocks + (size_t)r * P.L.bytes);
-    for (size_t i = threadIdx.x; i < n16; i += blockDim.x) {
-        lds_block[i] = g[i];
-    }
-    if (threadIdx.x == 0) {
-        lds_params = P;
-    }
-    __syncthreads();
-    sweep_replica_on(lds_engine, lds_params, r, (char*)lds_block, steps, rep_slot, 1);
-    __syncthreads();
-    for (size_t i = threadIdx.x; i < n16; i += blockDim.x) {
-        g[i] = lds_block[i];
     }
 }
 
@@ -294,34 +252,6 @@ extern "C" __global__ void ldo_batch_init_kernel(const Params* plist, int32_t n,
     const int32_t* h = cfg + m.off;
     int nc = m.n_chains, nd = m.n_domains;
     init_replica(plist[k], 0, h, h + nc, h + 2 * nc, h + 2 * nc + 3 * nd, nc, 0, nullptr);
-}
-
-// One workgroup per chain with the chain's block, its parameters and the
-// engine object in LDS (dynamic LDS = the largest block of the batch).
-extern "C" __global__ void __launch_bounds__(64)
-    ldo_batch_sweep_lds_kernel(const Params* plist, int32_t n, int64_t steps) {
-    extern __shared__ uint4 lds_block[];
-    __shared__ Params lds_params;
-    __shared__ Eng lds_engine;
-    int k = blockIdx.x;
-    if (k >= n) {
-        return;
-    }
-    if (threadIdx.x == 0) {
-        lds_params = plist[k];
-    }
-    __syncthreads();
-    size_t n16 = (size_t)lds_params.L.bytes / 16;
-    uint4* g = (uint4*)lds_params.blocks;
-    for (size_t i = threadIdx.x; i < n16; i += blockDim.x) {
-        lds_block[i] = g[i];
-    }
-    __syncthreads();
-    sweep_replica_on(lds_engine, lds_params, 0, (char*)lds_block, steps, nullptr, 1);
-    __syncthreads();
-    for (size_t i = threadIdx.x; i < n16; i += blockDim.x) {
-        g[i] = lds_block[i];
-    }
 }
 
 // Blocks in device memory: mode 0, one chain per wavefront run by all its
@@ -569,13 +499,14 @@ void choose_sweep_kernel(Ctx& c) {
     hip_check(hipDeviceGetAttribute(&optin, hipDeviceAttributeSharedMemPerBlockOptin, dev),
               "shared memory opt-in limit");
     hipFuncAttributes fa;
-    hip_check(hipFuncGetAttributes(&fa, (const void*)ldo_sweep_lds_kernel), "kernel attributes");
-    size_t need = (size_t)c.P.L.bytes + fa.sharedSizeBytes;
+    hip_check(hipFuncGetAttributes(&fa, (const void*)wave_kernels(c.P).sweep), "kernel attributes");
+    size_t need = (size_t)wave_lds_bytes(c.P) + fa.sharedSizeBytes;
     if (optin <= 0 || need > (size_t)optin) {
         return;
     }
-    hip_check(hipFuncSetAttribute((const void*)ldo_sweep_lds_kernel,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)c.P.L.bytes),
+    hip_check(hipFuncSetAttribute((const void*)wave_kernels(c.P).sweep,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)wave_lds_bytes(c.P)),
               "dynamic LDS size");
     c.lds_sweep = true;
 }
@@ -593,8 +524,9 @@ void launch_sweep(Ctx& c, int64_t steps, const int32_t* rep_slot) {
     const int32_t* q_to_rep = rep_slot != nullptr ? c.d_xint : nullptr;
     launch_timed(c, 0, [&]() {
         if (c.lds_sweep) {
-            hipLaunchKernelGGL(ldo_sweep_lds_kernel, dim3(c.R), dim3(64), (size_t)c.P.L.bytes,
-                               c.stream, c.P, steps, rep_slot, q_to_rep);
+            hipLaunchKernelGGL(wave_kernels(c.P).sweep, dim3(c.R), dim3(64),
+                               (size_t)wave_lds_bytes(c.P), c.stream, c.P, steps, rep_slot,
+                               q_to_rep);
         }
         else {
             hipLaunchKernelGGL(ldo_sweep_kernel, grid_of(c), dim3(64), 0, c.stream, c.P, steps,
@@ -1379,8 +1311,9 @@ struct BatchCtx {
     int32_t* d_cfg = nullptr;
     BatchCfg* d_meta = nullptr;
     RepScalars* d_scalars = nullptr;
-    size_t max_block = 0;
+    size_t max_lds = 0;
     bool lds_ok = false;
+    BatchSweepFn lds_kernel = nullptr;
     int kernel = LDO_BATCH_WAVE;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
 };
@@ -1478,7 +1411,7 @@ void batch_check(BatchCtx& b) {
 double batch_launch(BatchCtx& b, int kernel, int64_t steps) {
     hip_check(hipEventRecord(b.ev0, b.stream), "event record");
     if (kernel == LDO_BATCH_LDS) {
-        hipLaunchKernelGGL(ldo_batch_sweep_lds_kernel, dim3(b.n), dim3(64), b.max_block, b.stream,
+        hipLaunchKernelGGL(b.lds_kernel, dim3(b.n), dim3(64), b.max_lds, b.stream,
                            b.d_params, b.n, steps);
     }
     else if (kernel == LDO_BATCH_WAVE || kernel == LDO_BATCH_WAVE_SOLO) {
@@ -1539,7 +1472,10 @@ int ldo_batch_create(int32_t n_chains, const ldo_system_desc* systems, const ldo
             tident.insert(tident.end(), pl.type_ident.begin(), pl.type_ident.end());
             block_off[k] = blocks;
             blocks += (size_t)pl.P.L.bytes;
-            b->max_block = std::max(b->max_block, (size_t)pl.P.L.bytes);
+            b->max_lds = std::max(b->max_lds, (size_t)wave_lds_bytes(pl.P));
+            if (b->lds_kernel == nullptr || wave_all_kinds(pl.P)) {
+                b->lds_kernel = wave_kernels(pl.P).batch;
+            }
             std::vector<int32_t> h;
             int nd = 0;
             try {
@@ -1600,12 +1536,12 @@ int ldo_batch_create(int32_t n_chains, const ldo_system_desc* systems, const ldo
         hip_check(hipDeviceGetAttribute(&optin, hipDeviceAttributeSharedMemPerBlockOptin, dev),
                   "shared memory opt-in limit");
         hipFuncAttributes fa;
-        hip_check(hipFuncGetAttributes(&fa, (const void*)ldo_batch_sweep_lds_kernel),
+        hip_check(hipFuncGetAttributes(&fa, (const void*)b->lds_kernel),
                   "kernel attributes");
-        if (optin > 0 && b->max_block + fa.sharedSizeBytes <= (size_t)optin) {
-            hip_check(hipFuncSetAttribute((const void*)ldo_batch_sweep_lds_kernel,
+        if (optin > 0 && b->max_lds + fa.sharedSizeBytes <= (size_t)optin) {
+            hip_check(hipFuncSetAttribute((const void*)b->lds_kernel,
                                           hipFuncAttributeMaxDynamicSharedMemorySize,
-                                          (int)b->max_block),
+                                          (int)b->max_lds),
                       "dynamic LDS size");
             b->lds_ok = true;
             b->kernel = LDO_BATCH_LDS;

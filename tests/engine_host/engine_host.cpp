@@ -71,6 +71,24 @@ void learned_replica(const Params& P, int r, int64_t attempts) {
     }
 }
 
+// One replica's sweep as the library picks its kernel: the wavefront engine on
+// a staged copy of the block with a wavefront per replica, else (or with
+// LDO_SWEEP_KERNEL=global) the general engine on the block itself.
+void sweep_one(const HostCtx& c, int r, int64_t steps, const int32_t* rep_slot) {
+    const char* force = std::getenv("LDO_SWEEP_KERNEL");
+    bool global = force != nullptr && std::strcmp(force, "global") == 0;
+    if (global || c.P.lanes_per_replica != 64) {
+        sweep_replica(c.P, r, steps, rep_slot);
+        return;
+    }
+    char* blk = c.blocks + (size_t)r * c.P.L.bytes;
+    std::vector<uint4> lds((size_t)wave_lds_bytes(c.P) / 16);
+    std::memcpy((char*)lds.data(), blk, (size_t)c.P.L.stage);
+    auto sweep = wave_all_kinds(c.P) ? sweep_wave<true> : sweep_wave<false>;
+    sweep(c.P, r, blk, (char*)lds.data(), steps, rep_slot);
+    std::memcpy(blk, (char*)lds.data(), (size_t)c.P.L.stage);
+}
+
 void set_tables(HostCtx& c) {
     int n = c.R;
     size_t n2 = (size_t)c.plan.spec.n_ident * c.plan.spec.n_ident;
@@ -343,7 +361,7 @@ int eh_sweep(void* ctx, int64_t steps) {
             throw ldo::AbiError {LDO_E_ARG, "negative step count"};
         }
         for (int r = 0; r < c->R; r++) {
-            sweep_replica(c->P, r, steps, nullptr);
+            sweep_one(*c, r, steps, nullptr);
         }
         check_statuses(*c);
     });
@@ -449,7 +467,7 @@ int eh_run(void* ctx, int64_t n_swaps, int64_t interval) {
             int64_t rng_ctr = ++c->swap_counter;
             int64_t swap_i = rng_ctr - c->swap_base;
             for (int r = 0; r < c->R; r++) {
-                sweep_replica(c->P, r, interval, X.rep_slot);
+                sweep_one(*c, r, interval, X.rep_slot);
             }
             if (c->P.exchange_mode == LDO_EXCHANGE_WINDOWS) {
                 exchange_windows_round(c->P, X, swap_i, rng_ctr);
@@ -484,7 +502,7 @@ int eh_exchange(void* ctx, int64_t swap_index) {
         int64_t rng_ctr = ++c->swap_counter;
         // update_control_qs and update_dependent_qs: an interval of 0 steps
         for (int r = 0; r < c->R; r++) {
-            sweep_replica(c->P, r, 0, X.rep_slot);
+            sweep_one(*c, r, 0, X.rep_slot);
         }
         if (c->P.exchange_mode == LDO_EXCHANGE_WINDOWS) {
             exchange_windows_round(c->P, X, swap_index, rng_ctr);

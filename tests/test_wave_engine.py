@@ -1,0 +1,107 @@
+"""The wavefront sweep engine at the forms where it leaves the general one:
+rings (segments and stacked pairs across the scaffold's ends), sequence
+specific stacking (energies that differ from pair to pair), disallowed
+misbinding, more staples than a wavefront has lanes, staples of up to eight
+domains in strides with unused slots, and centring and constraint checks every
+few steps.  Each runs step for step against the CPU oracle, on the host build
+of the engine and on the GPU, and the general engine runs beside it."""
+import dataclasses
+import os
+
+import pytest
+
+import parity_cases as pc
+from test_engine_host_parity import sampler_cls as host_sampler  # noqa: F401
+from latticednaorigami_amd import abi, systems
+
+RING = [(0, 0, 0), (1, 0, 0), (2, 0, 0), (3, 0, 0), (3, 1, 0), (2, 1, 0), (1, 1, 0), (0, 1, 0)]
+
+
+def ring(domain_type, moves):
+    s = systems.four_domain_system(max_total_staples=8)
+    n = len(RING)
+    return dataclasses.replace(
+        s, identities=[[-(i + 1) for i in range(n)], [1, 2], [3, 6], [4, 5], [7, 8], [8, 1]],
+        chains=[systems.Chain(0, 0, RING, [(0, 0, 1)] * n)], cyclic=True,
+        domain_type=domain_type, moves=moves(n), temps=[335.0, 348.0])
+
+
+def raster(**kw):
+    s = systems.raster_system(n_domains=20, width=5, replicas=2, t_lo=325.0, t_hi=345.0)
+    return dataclasses.replace(s, **kw)
+
+
+def crowded():
+    """A concentration at which more than 64 staples hang on four domains
+    (without scaffold regrowth, whose growth stack holds 32 levels)."""
+    s = systems.four_domain_system(max_total_staples=160)
+    moves = [systems.Move(abi.MOVE_ORIENTATION_ROTATION, 0.1),
+             systems.Move(abi.MOVE_MET_STAPLE_EXCHANGE, 0.7),
+             systems.Move(abi.MOVE_CB_STAPLE_REGROWTH, 0.2)]
+    return dataclasses.replace(s, staple_M=3000.0, max_type_staples=160, moves=moves,
+                               temps=[320.0, 350.0])
+
+
+def long_staples(moves):
+    s = systems.four_domain_system(max_total_staples=6)
+    n = 12
+    return dataclasses.replace(
+        s, identities=[[-(i + 1) for i in range(n)], [1, 2, 3, 4, 5, 6, 7, 8], [9, 10, 11],
+                       [12, 11, 3], [5]],
+        chains=[systems.Chain(0, 0, [(i, 0, 0) for i in range(n)], [(0, 0, 1)] * n)],
+        max_staple_size=8, staple_M=1e-3, moves=moves(n), temps=[340.0, 360.0],
+        flags=abi.FLAG_CTCB_SCAFFOLD_ENDPOINTS)
+
+
+FORMS = {
+    "ring": lambda: ring(abi.HALFTURN, systems.standard_moveset),
+    "ring_three_quarter": lambda: ring(abi.THREEQUARTERTURN, systems.standard_moveset),
+    "ring_ctrg": lambda: ring(abi.HALFTURN, systems.ctrg_moveset),
+    "ring_jump": lambda: ring(abi.THREEQUARTERTURN, systems.jump_moveset),
+    "sequence_stacking": lambda: raster(stacking_pot=abi.STACK_SEQUENCESPECIFIC),
+    "sequence_stacking_ctrg": lambda: raster(stacking_pot=abi.STACK_SEQUENCESPECIFIC,
+                                             moves=systems.ctrg_moveset(12)),
+    "misbinding_disallowed": lambda: raster(misbinding_pot=abi.MISBIND_DISALLOWED),
+    "crowded": crowded,
+    "long_staples": lambda: long_staples(systems.standard_moveset),
+    "long_staples_ctrg": lambda: long_staples(systems.ctrg_moveset),
+    "centred": lambda: raster(centering_freq=7, constraint_check_freq=11),
+}
+
+
+def check(make, oracle_mod, name):
+    s = FORMS[name]()
+    print("form", name, flush=True)
+    steps = 4000 if name == "crowded" else 150 if "ctrg" in name or "jump" in name else 1500
+    os.environ["LDO_SWEEP_KERNEL"] = "global"
+    try:
+        general = make(s, temps=s.temps)
+        general.sweep(steps)
+    finally:
+        del os.environ["LDO_SWEEP_KERNEL"]
+    wave = make(s, temps=s.temps)
+    ref = oracle_mod.Oracle(s, temps=s.temps)
+    for k in range(3):
+        wave.sweep(steps)
+        ref.sweep(steps)
+        for r in range(len(s.temps)):
+            pc.assert_same(wave, ref, r)
+            if k == 0:
+                pc.assert_same(general, ref, r)
+                assert wave.move_tracking(r) == general.move_tracking(r)
+    pc.assert_counters(wave, ref)
+    return wave
+
+
+@pytest.mark.parametrize("name", sorted(FORMS))
+def test_forms_on_the_host_build(host_sampler, oracle_mod, name):  # noqa: F811
+    wave = check(host_sampler, oracle_mod, name)
+    if name == "crowded":
+        assert max(wave.observables(r)["num_staples"] for r in range(2)) > 64
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", sorted(FORMS))
+def test_forms_on_the_gpu(oracle_mod, name):
+    from latticednaorigami_amd.sampler import Sampler
+    check(Sampler, oracle_mod, name)

@@ -1314,6 +1314,18 @@ struct BatchCtx {
     size_t max_lds = 0;
     bool lds_ok = false;
     BatchSweepFn lds_kernel = nullptr;
+    // The LDS sweep's launches: chains by decreasing LDS need, cut where fewer
+    // or more of them fit a CU, each group on a stream of its own (one launch
+    // would give every chain the largest one's LDS: three to a CU instead of
+    // the mean's six at 8 to 128 domains).
+    struct Group {
+        int first, count;
+        size_t lds;
+    };
+    std::vector<Group> groups;
+    std::vector<hipStream_t> side;   // streams of the groups after the first
+    std::vector<hipEvent_t> side_ev;
+    int32_t* d_order = nullptr;
     int kernel = LDO_BATCH_WAVE;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
 };
@@ -1378,6 +1390,13 @@ void free_batch(BatchCtx* b) {
     bfree(b->d_cfg);
     bfree(b->d_meta);
     bfree(b->d_scalars);
+    bfree(b->d_order);
+    for (hipEvent_t e: b->side_ev) {
+        (void)hipEventDestroy(e);
+    }
+    for (hipStream_t st: b->side) {
+        (void)hipStreamDestroy(st);
+    }
     if (b->ev0) {
         (void)hipEventDestroy(b->ev0);
     }
@@ -1408,11 +1427,59 @@ void batch_check(BatchCtx& b) {
 
 // Launches `steps` steps on every chain with the batch's sweep kernel and
 // returns the kernel time.
+// The groups of the LDS sweep (BatchCtx::groups).
+void group_batch(BatchCtx& b) {
+    std::vector<int32_t> order(b.n);
+    std::vector<size_t> lds(b.n);
+    for (int k = 0; k < b.n; k++) {
+        order[k] = k;
+        lds[k] = (size_t)wave_lds_bytes(b.params[k]);
+    }
+    std::stable_sort(order.begin(), order.end(),
+                     [&](int32_t x, int32_t y) { return lds[x] > lds[y]; });
+    int dev = 0, cus = 0, per_cu = 0;
+    hip_check(hipGetDevice(&dev), "get device");
+    hip_check(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), "CUs");
+    hip_check(hipDeviceGetAttribute(&per_cu, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor,
+                                    dev), "LDS of a CU");
+    // chains of this LDS need that fit a CU, in steps of two up to the eight
+    // wavefronts its registers hold; a batch that fits at once is one group
+    auto fit = [&](size_t need) { return std::min<size_t>(8, std::max<size_t>(1, per_cu / need)); };
+    bool whole = (size_t)b.n <= fit(b.max_lds) * cus;
+    for (int i = 0; i < b.n; i++) {
+        size_t need = lds[order[i]];
+        if (b.groups.empty() || (!whole && fit(need) / 2 > fit(b.groups.back().lds) / 2)) {
+            b.groups.push_back({i, 0, need});
+        }
+        b.groups.back().count++;
+    }
+    b.side.resize(b.groups.size() - 1);
+    b.side_ev.resize(b.groups.size() - 1);
+    for (size_t g = 0; g + 1 < b.groups.size(); g++) {
+        hip_check(hipStreamCreate(&b.side[g]), "stream");
+        hip_check(hipEventCreateWithFlags(&b.side_ev[g], hipEventDisableTiming), "event create");
+    }
+    bupload(b, b.d_order, order, "copy order");
+}
+
 double batch_launch(BatchCtx& b, int kernel, int64_t steps) {
     hip_check(hipEventRecord(b.ev0, b.stream), "event record");
     if (kernel == LDO_BATCH_LDS) {
-        hipLaunchKernelGGL(b.lds_kernel, dim3(b.n), dim3(64), b.max_lds, b.stream,
-                           b.d_params, b.n, steps);
+        for (size_t g = 0; g < b.groups.size(); g++) {
+            hipStream_t st = g == 0 ? b.stream : b.side[g - 1];
+            if (g > 0) {
+                hip_check(hipStreamWaitEvent(st, b.ev0, 0), "fork");
+            }
+            hipLaunchKernelGGL(b.lds_kernel, dim3(b.groups[g].count), dim3(64), b.groups[g].lds, st,
+                               b.d_params, b.d_order + b.groups[g].first, b.groups[g].count, steps);
+            hip_check(hipGetLastError(), "launch batch sweep");
+            if (g > 0) {
+                hip_check(hipEventRecord(b.side_ev[g - 1], st), "event record");
+            }
+        }
+        for (hipEvent_t e: b.side_ev) {
+            hip_check(hipStreamWaitEvent(b.stream, e, 0), "join");
+        }
     }
     else if (kernel == LDO_BATCH_WAVE || kernel == LDO_BATCH_WAVE_SOLO) {
         hipLaunchKernelGGL(ldo_batch_sweep_kernel, dim3(b.n), dim3(64), 0, b.stream, b.d_params,
@@ -1543,6 +1610,7 @@ int ldo_batch_create(int32_t n_chains, const ldo_system_desc* systems, const ldo
                                           hipFuncAttributeMaxDynamicSharedMemorySize,
                                           (int)b->max_lds),
                       "dynamic LDS size");
+            group_batch(*b);
             b->lds_ok = true;
             b->kernel = LDO_BATCH_LDS;
         }

@@ -9,7 +9,7 @@
 #include "replica_ops.h"
 
 typedef void (*SweepFn)(Params, int64_t, const int32_t*, const int32_t*);
-typedef void (*BatchSweepFn)(const Params*, int32_t, int64_t);
+typedef void (*BatchSweepFn)(const Params*, const int32_t*, int32_t, int64_t);
 struct WaveKernels {
     SweepFn sweep;
     BatchSweepFn batch;
@@ -65,16 +65,17 @@ __global__ void __launch_bounds__(64)
     sweep_staged<ALL>(P, r, P.blocks + (size_t)r * P.L.bytes, (lds_t)lds_block, steps, rep_slot);
 }
 
-// One wavefront per chain with the wavefront engine (dynamic LDS = the
-// largest wave_lds_bytes of the batch).
+// One wavefront per chain of `order` (n of them) with the wavefront engine;
+// dynamic LDS = the largest wave_lds_bytes of these chains.
 template <bool ALL>
 __global__ void __launch_bounds__(64)
-    ldo_batch_sweep_lds_kernel(const Params* plist, int32_t n, int64_t steps) {
+    ldo_batch_sweep_lds_kernel(const Params* plist, const int32_t* order, int32_t n,
+                               int64_t steps) {
     extern __shared__ uint4 lds_block[];
-    int k = blockIdx.x;
-    if (k >= n) {
+    if ((int)blockIdx.x >= n) {
         return;
     }
+    int k = uni(order[blockIdx.x]);
     // nothing writes the parameters during a launch: scalar loads
     const Params& P = *(const Params*)(__attribute__((address_space(4))) const Params*)(plist + k);
     sweep_staged<ALL>(P, 0, P.blocks, (lds_t)lds_block, steps, nullptr);

@@ -432,6 +432,8 @@ struct Eng {
     DEV bool agreed(bool b) const { return b; }
     DEV void rng_begin() { S->rng_idx = 0; }
     DEV bool all_kinds() const { return true; }
+    DEV int kind_of(int m) const { return P->move_kind[m]; }
+    DEV int maxreg_of(int m) const { return P->move_maxreg[m]; }
     DEV void rg_look(const RgCur&) {}
     DEV int staple_of(int k) const { return ((const int16_t*)sframes)[k]; }
     // prev[s] = the domain's position and orientation

@@ -598,7 +598,8 @@ struct FourBody {
 // when no lane has a candidate for one.  Positions are folded into one word
 // (x + 2^10 y + 2^20 z): every difference taken is one of chain neighbours',
 // a unit vector.  HALF: HalfTurn domains, whose twist rule is that contiguous
-// domains off the orientation's axis point in opposite directions.
+// domains off the orientation's axis point in opposite directions.  ONE: every
+// pair has the same stacking energy, so a term's pairs are not told.
 struct FbTerm {
     int op;         // 0 none; 1 + s1; 2 - s1; 3 - s1/2 - s2/2; 4 - s1 - s2
     int viol;
@@ -624,7 +625,7 @@ DEV int fb_index(int d) {
     return 2 * (m > 1) + 2 * (m > 1024) + (d < 0);
 }
 
-template <class A, bool HALF>
+template <class A, bool HALF, bool ONE>
 struct FbChecks {
     const A& a; // rec(s) as a record, ns, lmask, cyc
     DEV explicit FbChecks(const A& acc) : a(acc) {}
@@ -709,13 +710,21 @@ struct FbChecks {
             out.helix = is_p & live & helix;
             out.viol = is_p & live & ((contig & !ahead) | (helix & turn) | (!next_to & !kink));
             out.op = is_p & pair_on & !contig & !central;
-            out.a1 = p;
-            out.b1 = q;
+            if (!ONE) {
+                out.a1 = p;
+                out.b1 = q;
+            }
         }
         // what is kept of it: one word instead of a lane mask each
         enum { ON = 1, CONTIG_PAIR = 2, OFF_STACK = 4, NEXT_TO = 8, STACKED = 16, LIVE = 32 };
         int kind = keep((int)pair_on * ON | (int)contig * CONTIG_PAIR | (int)central * OFF_STACK |
                         (int)next_to * NEXT_TO | (int)spq * STACKED | (int)live * LIVE);
+        t = keep(t); // the kinds of check below are worked out again from it
+        back = keep(back);
+        is_j = (unsigned)(t - 1) < 9u;
+        is_t = (unsigned)(t - 10) < 3u;
+        is_c = t == 14;
+        is_tail = (t == 13) & (back != 0);
         // n: the end the check leaves from; f: the other
         bool leave = (is_j & ((kind & (CONTIG_PAIR | OFF_STACK)) == 0)) | is_t;
         bool fw = is_tail | (leave & (back == 0));
@@ -726,7 +735,7 @@ struct FbChecks {
         nb = is_c ? dj : nb;
         int nf = fwd(nb), nr = bwd(nb);
         FbWord ro = rec(far), rnb = rec(nb), rnf = rec(nf), rnr = rec(nr);
-        int i = is_j ? (t >= 4) + (t >= 7) : (is_t ? t - 10 : 0);
+        int i = keep(is_j ? (t >= 4) + (t >= 7) : (is_t ? t - 10 : 0));
         int v;
         {
             // the outer candidates after far, which a junction restricts
@@ -762,6 +771,11 @@ struct FbChecks {
         }
         bool bv = bound(rv, v);
         bool sv = stacked(u, ru, v, rv);
+        t = keep(t);
+        back = keep(back);
+        is_t = (unsigned)(t - 10) < 3u;
+        is_c = t == 14;
+        is_tail = (t == 13) & (back != 0);
         {
             // ---- triplets (v, n, f)
             bool bk = (is_t & (back != 0)) | (is_c & (second == 0));
@@ -785,13 +799,16 @@ struct FbChecks {
             int nv = is_c ? dj : n, nl = is_t & (i == 2) ? nb : n;
             bool any_t = trip & (t != 0);
             out.op = any_t ? (both ? 3 : (lone_v | lone_f ? 2 : 0)) : out.op;
-            out.a1 = any_t ? (both ? (bk ? v : f) : (lone_v ? nv : nl)) : out.a1;
-            out.b1 = any_t ? (both ? n : (lone_v ? v : f)) : out.b1;
-            out.a2 = n;
-            out.b2 = bk ? f : v;
+            if (!ONE) {
+                out.a1 = any_t ? (both ? (bk ? v : f) : (lone_v ? nv : nl)) : out.a1;
+                out.b1 = any_t ? (both ? n : (lone_v ? v : f)) : out.b1;
+                out.a2 = n;
+                out.b2 = bk ? f : v;
+            }
             out.viol = out.viol | (int)chain;
         }
         // ---- junctions
+        is_j = (unsigned)(keep(t) - 1) < 9u;
         bool off = (kind & (CONTIG_PAIR | OFF_STACK)) == 0; // out of a stacked pair's end
         bool ct = (kind & CONTIG_PAIR) != 0;
         bool jn_ok = is_j & ((kind & ON) != 0) & bv & !(off & sv);
@@ -828,10 +845,12 @@ struct FbChecks {
         int jop = n1 == n3 ? 4 : (n1 == -n3 ? 0 : 3);
         out.viol = jn_ok ? (int)jv : out.viol;
         out.op = jn_ok ? (jv ? 0 : jop) : out.op;
-        out.a1 = jn_ok ? (flip ? y : j1) : out.a1;
-        out.b1 = jn_ok ? (flip ? x : j2) : out.b1;
-        out.a2 = jn_ok ? (flip ? j2 : x) : out.a2;
-        out.b2 = jn_ok ? (flip ? j1 : y) : out.b2;
+        if (!ONE) {
+            out.a1 = jn_ok ? (flip ? y : j1) : out.a1;
+            out.b1 = jn_ok ? (flip ? x : j2) : out.b1;
+            out.a2 = jn_ok ? (flip ? j2 : x) : out.a2;
+            out.b2 = jn_ok ? (flip ? j1 : y) : out.b2;
+        }
         return out;
     }
     // v as one register (a wavefront's conditions are pairs of scalar

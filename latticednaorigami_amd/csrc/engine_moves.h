@@ -1018,7 +1018,6 @@ DEVNI int LDO_ENG::ctcb_staples() {
     }
     return nst;
 }
-#endif // LDO_WAVE
 
 // CTCBRegrowthMCMovetype::grow_chain (cb_movetypes.cpp:463-484) and
 // grow_staple_and_update_endpoints (:541-562), interleaved through an
@@ -1138,6 +1137,7 @@ DEVNI void LDO_ENG::ctcb_grow_chain_scaffold(int first, int count, int dir, bool
         sp--;
     }
 }
+#endif // LDO_WAVE
 
 // CTRegrowthMCMovetype::select_indices (movetypes.cpp:469-510): the
 // segment first, first + dir, ... (count domains), and the active endpoint
@@ -1979,7 +1979,7 @@ DEVNI bool LDO_ENG::ctcb_jump_move(int max_regrowth) {
 // MCMovetype::attempt_move and the reset_internal chain (movetypes.cpp:41-51,
 // 242-250; met_movetypes.cpp:45-48, 139-143; cb_movetypes.cpp:44-50, 457-461)
 DEVIN bool LDO_ENG::attempt(int m) {
-    return attempt_kind(P->move_kind[m], P->move_maxreg[m], m);
+    return attempt_kind(kind_of(m), maxreg_of(m), m);
 }
 
 DEVNI bool LDO_ENG::attempt_kind(int kind, int max_regrowth, int m) {

@@ -245,16 +245,16 @@ static __host__ __device__ __noinline__ FbOut wave_fb_walk(FbArgs g, int di, int
 
 // The walk's checks side by side (FbChecks).  On a violation e and st are not
 // set.
-template <bool HALF>
+template <bool HALF, bool ONE>
 static __host__ __device__ __noinline__ FbOut wave_fb_terms(FbArgs g, int di, int dj) {
     g = fb_uniform(g);
     FbLane a {g.dom, g.ns, g.flags & 255, (g.flags >> 8) & 1, (g.flags >> 9) & 1};
-    typedef FbChecks<FbLane, HALF> Checks;
+    typedef FbChecks<FbLane, HALF, ONE> Checks;
     Checks f(a);
     di = uni(di);
     dj = uni(dj);
     FbOut out {0.0, 0, 0};
-    bool one = ((g.flags >> 10) & 1) != 0;
+    constexpr bool one = ONE;
 #ifdef __HIP_DEVICE_COMPILE__
     int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
     FbTerm t = f.check(lane, di, dj,
@@ -423,6 +423,9 @@ struct WEng {
     uint64_t six_empty, six_unb, six_full;
     uint64_t six_walk;        // sites d's walks remain possible from
     uint64_t six_ends;        // sites that are an endpoint of d
+    // lane m: kind, max_regrowth and first tracking counters of move m, its
+    // attempts and accepts since the launch
+    int mv_kind, mv_maxreg, mv_track, mv_width, mv_att, mv_acc;
     // random draws of the current block of 64 (this lane's)
     uint64_t rng_draw;
     int rng_block;
@@ -775,7 +778,11 @@ struct WEng {
         }
 #endif
         FbArgs g {dom.p, dident.p, t_stack, stack_all, fb_flags, ns, n_ident};
-        FbOut o = dtype == 0 ? wave_fb_terms<true>(g, di, dj) : wave_fb_terms<false>(g, di, dj);
+        FbOut o = (fb_flags >> 10) & 1
+                      ? (dtype == 0 ? wave_fb_terms<true, true>(g, di, dj)
+                                    : wave_fb_terms<false, true>(g, di, dj))
+                      : (dtype == 0 ? wave_fb_terms<true, false>(g, di, dj)
+                                    : wave_fb_terms<false, false>(g, di, dj));
         o.st = uni(o.st);
         o.viol = uni(o.viol);
         if (o.viol && !trial) {
@@ -1148,13 +1155,22 @@ struct WEng {
 #include "engine_decl.h"
 
 #ifdef __HIP_DEVICE_COMPILE__
+    __device__ __forceinline__ void count_moves();
     __device__ __forceinline__ void look_six(int d, I3 pp);
-    __device__ __forceinline__ void walk_six(int d);
+    // sg, std_: seg[d] and stem[d]
+    __device__ __forceinline__ void walk_six(int d, int sg, int std_);
 #endif
     DEV bool agreed(bool b) const { return all_lanes(b); }
     // whether the moveset holds a recoil-growth or jump move: a constant of
     // the kernel, so that the kernels of the standard moveset leave their code out
     bool kinds;
+#ifdef __HIP_DEVICE_COMPILE__
+    __device__ __forceinline__ int kind_of(int m) const { return lane_int(mv_kind, m); }
+    __device__ __forceinline__ int maxreg_of(int m) const { return lane_int(mv_maxreg, m); }
+#else
+    DEV int kind_of(int m) const { return P->move_kind[m]; }
+    DEV int maxreg_of(int m) const { return P->move_maxreg[m]; }
+#endif
     DEVIN void rg_look(const RgCur& c);
     DEV bool all_kinds() const { return kinds; }
     DEV int staple_of(int k) const { return LArr<int16_t> {sframes.p}[k]; }
@@ -1348,13 +1364,134 @@ DEVIN bool WEng::rg_test_open(double p) {
     return all_lanes(p > uniform_real());
 }
 
+// ------------------------------------------------------------- CTCB growth
+// Eng::ctcb_grow_chain_scaffold with the level being grown in registers: the
+// stack in LDS is touched when a staple is entered or left.
+DEVNI void WEng::ctcb_grow_chain_scaffold(int first, int count, int dir, bool first_gp) {
+    int sp = 0;
+    GrowFrame f;
+    f.first = (int16_t)first;
+    f.count = (int16_t)count;
+    f.i = 1;
+    f.prev = (int16_t)first;
+    f.gold = 0;
+    f.gnew = 0;
+    f.dir = (int8_t)dir;
+    f.kind = 0;
+    f.phase = 0;
+    f.pad = 0;
+    bool have = count > 1;
+    int enter = -1; // growthpoint to descend at
+    if (first_gp && gp[first] >= 0) {
+        enter = first;
+    }
+    while (S->status == ST_OK && !S->rejected) {
+        if (enter >= 0) {
+            if (have) {
+                if (sp + 1 >= LDO_GROW_DEPTH) {
+                    fail(ST_CAPACITY);
+                    break;
+                }
+                gstack[sp++] = f;
+            }
+            have = true;
+            f.gold = (int16_t)enter;
+            f.kind = 1;
+            f.phase = 0;
+            enter = -1;
+        }
+        if (!have) {
+            if (sp == 0) {
+                break;
+            }
+            LGrowFrame g = gstack[--sp];
+            f.first = g.first;
+            f.count = g.count;
+            f.i = g.i;
+            f.prev = g.prev;
+            f.gold = g.gold;
+            f.gnew = g.gnew;
+            f.dir = g.dir;
+            f.kind = g.kind;
+            f.phase = g.phase;
+            have = true;
+        }
+        if (f.kind == 0) {
+            if (f.i >= f.count) {
+                have = false;
+                continue;
+            }
+            int d = walk(f.prev, f.dir);
+            int sd = seg[d], gd = gp[d], ed = inact[d];
+            if (sd < 0) {
+                seg[d] = 0; // get_dir's map insertion (top_constraint_points.cpp:179-185)
+            }
+            cb_select_and_set(d, f.prev);
+            if (S->rejected) {
+                break;
+            }
+            cp_remove_active(d);
+            if (ed >= 0) {
+                cp_add_active(ed, pos(d), seg[ed]);
+            }
+            f.prev = (int16_t)d;
+            f.i++;
+            enter = gd >= 0 ? d : -1;
+            continue;
+        }
+        // staple growth from growthpoint f.gold: the growthpoint itself, then
+        // the two ways from it
+        if (f.phase == 2) {
+            have = false;
+            continue;
+        }
+        if (f.phase == 0) {
+            int gnew = gp[f.gold];
+            if (cslot_of(gnew) == 0) {
+                have = false;
+                continue;
+            }
+            if (S->regrow_old) {
+                cb_set_old_growth_point(gnew, f.gold);
+            }
+            else {
+                double de = set_growth_point(gnew, f.gold);
+                S->bias *= exp(-de);
+            }
+            if (S->rejected) {
+                break;
+            }
+            cp_update_endpoints(gnew);
+            f.gnew = (int16_t)gnew;
+        }
+        int di = d_of(f.gnew);
+        int n = f.phase == 0 ? ch[cslot_of(f.gnew)].len - di : di + 1;
+        int way = f.phase == 0 ? 1 : -1;
+        f.phase++;
+        if (n > 1) {
+            if (sp + 1 >= LDO_GROW_DEPTH) {
+                fail(ST_CAPACITY);
+                break;
+            }
+            gstack[sp++] = f;
+            f.first = f.gnew;
+            f.count = (int16_t)n;
+            f.i = 1;
+            f.prev = f.gnew;
+            f.dir = (int8_t)way;
+            f.kind = 0;
+            f.phase = 0;
+        }
+    }
+}
+
 // ------------------------------------------------------ CTRG configurations
 // the sites around the level's chain neighbour, before its attempts
 DEVIN void WEng::rg_look(const RgCur& c) {
 #ifdef __HIP_DEVICE_COMPILE__
     if (!c.stemd && six_d != c.d) {
         look_six(c.d, pos(c.ref));
-        walk_six(c.d);
+        walk_six(c.d, seg[c.d], stem[c.d]);
     }
 #endif
 }
@@ -1483,15 +1620,15 @@ __device__ __forceinline__ void WEng::look_six(int d, I3 pp) {
 // those that are an endpoint of d (cp_endpoint_reached): 64 endpoints are read
 // at once, and each that concerns d's chain and segment is held against all
 // six sites.
-__device__ __forceinline__ void WEng::walk_six(int d) {
+__device__ __forceinline__ void WEng::walk_six(int d, int sg, int std_) {
     int n = S->n_active;
     six_walk = ~0ull;
     six_ends = 0;
     if (n == 0) {
         return;
     }
-    int sg = seg[d], sg2 = -2, sw = sg;
-    if (stem[d] >= 0) {
+    int sg2 = -2, sw = sg;
+    if (std_ >= 0) {
         // a scaffold stem of a jump is held by its own pair of segments, any
         // other stem by none
         bool held = S->n_jsegs != 0 && cslot_of(d) == 0 && stemseg[d] >= 0;
@@ -1562,15 +1699,20 @@ __device__ __forceinline__ void WEng::walk_six(int d) {
 // that is no candidate adds zero).  d is unassigned: every grower unassigns
 // its domains first.
 DEVNI void WEng::cb_select_and_set(int d, int prev_d) {
-    FbRec pr = rec(prev_d);
-    I3 pp = i3(pr.x, pr.y, pr.z);
-    if (dom[d].state != OCC_UNASSIGNED) {
+    bool ctcb = S->kind == LDO_MOVE_KIND_CTCB;
+    // everything known of d and its neighbour, in one round of reads
+    uint4 q0 = *(LDO_LDS const uint4*)(dom.p + prev_d * 16);
+    int q1 = *(LDO_LDS const int8_t*)(dom.p + d * 16 + 13);
+    int q2 = dident.lane(d);
+    int q3 = seg.lane(d), q4 = stem.lane(d);
+    uint4 q5 = *(LDO_LDS const uint4*)(old.p + d * 16);
+    I3 pp = i3(uni((int32_t)q0.x), uni((int32_t)q0.y), uni((int32_t)q0.z));
+    int id = uni(q2);
+    if (uni(q1) != OCC_UNASSIGNED) {
         fail(ST_CONSTRAINT);
         S->rejected = 1;
         return;
     }
-    bool ctcb = S->kind == LDO_MOVE_KIND_CTCB;
-    int id = dident[d];
 #ifdef __HIP_DEVICE_COMPILE__
     int lane = plane();
     look_six(d, pp);
@@ -1613,7 +1755,7 @@ DEVNI void WEng::cb_select_and_set(int d, int prev_d) {
     }
     uint64_t weigh = mc;
     if (ctcb) {
-        walk_six(d);
+        walk_six(d, uni(q3), uni(q4));
         weigh &= six_walk;
         // an occupied site takes d only as an endpoint or of its own chain
         if (munb & weigh) {
@@ -1663,9 +1805,8 @@ DEVNI void WEng::cb_select_and_set(int d, int prev_d) {
         }
     }
     else {
-        LPosOre q = old[d];
-        p = i3(q.x, q.y, q.z);
-        o = q.ore;
+        p = i3(uni((int32_t)q5.x), uni((int32_t)q5.y), uni((int32_t)q5.z));
+        o = uni((int32_t)q5.w);
         uint64_t sel = ballot((six_p.x == p.x) & (six_p.y == p.y) & (six_p.z == p.z)) &
                        (mempty | munb | six_full);
         l = sel ? __builtin_ctzll(sel) : -1;
@@ -1687,6 +1828,8 @@ DEVNI void WEng::cb_select_and_set(int d, int prev_d) {
     }
     push_assigned(d);
 #else
+    (void)q3;
+    (void)q4;
     bool cand[6], unb[6];
     double wt[6], e1[6];
     int core[6], st1[6];
@@ -1747,9 +1890,8 @@ DEVNI void WEng::cb_select_and_set(int d, int prev_d) {
         }
     }
     else {
-        LPosOre q = old[d];
-        p = i3(q.x, q.y, q.z);
-        o = q.ore;
+        p = i3((int32_t)q5.x, (int32_t)q5.y, (int32_t)q5.z);
+        o = (int32_t)q5.w;
         for (int v = 0; v < 6; v++) {
             sel = eq3(p, add3(pp, unit3(v))) ? v : sel;
         }
@@ -1795,6 +1937,17 @@ DEVIN void WEng::cp_remove_active(int s, bool rec) {
         int i = base + plane();
         bool keep = false, drop = false;
         Endpoint e;
+#ifdef __HIP_DEVICE_COMPILE__
+        if (base == 0) {
+            // two words tell which go; mostly none does
+            LDO_LDS const int32_t* q = (LDO_LDS const int32_t*)(ep + i * (int)sizeof(Endpoint));
+            drop = (i < n) & (q[0] == (cs | dd << 16)) & (q[1] == sg);
+            if (ballot(drop) == 0) {
+                k = n < 64 ? n : 64;
+                continue;
+            }
+        }
+#endif
         if (i < n) {
             e = active_at(i);
             keep = !(e.cslot == cs && e.seg == sg && e.d == dd);
@@ -2017,54 +2170,64 @@ DEVNI void WEng::count_window_op() {
 }
 
 // ------------------------------------------------------------------- steps
+// Where the tracking counters of move kind `kind` begin (Layout::off_track)
+// and how far its accepts lie behind its attempts.
+DEV void track_range(const Layout& L, int kind, int& at, int& width) {
+    int T = L.ntypes, n1 = L.ns + 1, s1 = L.smax + 1;
+    at = kind == 2 ? 4 * T
+                   : (kind == 3 ? 6 * T
+                                : (kind == 4 ? 6 * T + 2 * n1 + 2 * s1
+                                             : (kind == 5 ? 6 * T + 4 * n1 + 2 * s1
+                                                          : 6 * T + 4 * n1 + 2 * s1 + 2)));
+    at = kind == 1 ? 0 : at;
+    width = kind <= 2 ? T : (kind == 5 ? 1 : (kind == 6 ? s1 : n1));
+}
+
 // Eng::track_move on the counters in device memory
 DEVIN void WEng::track_move(int m, bool acc) {
     S->last_move = m;
     S->last_acc = acc ? 1 : 0;
-    int T = P->L.ntypes, n1 = ns + 1, s1 = P->L.smax + 1;
+    int kind = kind_of(m), at, w;
+#ifdef __HIP_DEVICE_COMPILE__
+    at = lane_int(mv_track, m);
+    w = lane_int(mv_width, m);
+#else
+    track_range(P->L, kind, at, w);
+#endif
+    if (kind == 0 || (kind == 2 && S->trk_nost)) {
+        return;
+    }
     int64_t* t = (int64_t*)(gblk + P->L.off_track);
-    // attempts at i, accepts at i + w; a CTCB move counts a second pair
-    int i = -1, w = 0, i2 = -1;
-    switch (P->move_kind[m]) {
-    case 1:
-        i = (S->trk_ins ? 0 : 2 * T) + S->trk_type;
-        w = T;
-        break;
-    case 2:
-        i = S->trk_nost ? -1 : 4 * T + S->trk_type;
-        w = T;
-        break;
-    case 3:
-        i = 6 * T + S->trk_len;
-        w = n1;
-        i2 = 6 * T + 2 * n1 + S->trk_nst;
-        break;
-    case 4:
-        i = 6 * T + 2 * n1 + 2 * s1 + S->trk_len;
-        w = n1;
-        break;
-    case 5:
-        i = 6 * T + 4 * n1 + 2 * s1;
-        w = 1;
-        break;
-    case 6:
-        i = 6 * T + 4 * n1 + 2 * s1 + 2 + S->trk_nst;
-        w = s1;
-        break;
+    int key = kind == 1 ? (S->trk_ins ? 0 : 2 * w) + S->trk_type
+                        : (kind == 2 ? S->trk_type
+                                     : (kind == 5 ? 0 : (kind == 6 ? S->trk_nst : S->trk_len)));
+    wave_count(t + at + key, 1);
+    if (acc) {
+        wave_count(t + at + key + w, 1);
     }
-    if (i >= 0) {
-        wave_count(t + i, 1);
+    if (kind == 3) {
+        // a CTCB move counts its staples too
+        int64_t* u = t + at + 2 * w + S->trk_nst;
+        wave_count(u, 1);
         if (acc) {
-            wave_count(t + i + w, 1);
-        }
-    }
-    if (i2 >= 0) {
-        wave_count(t + i2, 1);
-        if (acc) {
-            wave_count(t + i2 + s1, 1);
+            wave_count(u + P->L.smax + 1, 1);
         }
     }
 }
+
+#ifdef __HIP_DEVICE_COMPILE__
+// the lanes' attempts and accepts to the block's counters
+__device__ __forceinline__ void WEng::count_moves() {
+    if (plane() < LDO_MAX_MOVES) {
+        LDO_LDS int64_t* a = (LDO_LDS int64_t*)S->attempts.p + plane();
+        LDO_LDS int64_t* c = (LDO_LDS int64_t*)S->accepts.p + plane();
+        *a += mv_att;
+        *c += mv_acc;
+    }
+    mv_att = 0;
+    mv_acc = 0;
+}
+#endif
 
 // GCMCSimulation::simulate (simulation.cpp:568-653) and select_movetype
 // (:655-665)
@@ -2074,7 +2237,13 @@ DEVNI void WEng::simulate(int64_t steps) {
     int64_t to_center = P->centering_freq > 0 ? P->centering_freq - S->step % P->centering_freq : 0;
     int64_t to_check = P->check_freq > 0 ? P->check_freq - S->step % P->check_freq : 0;
 #ifdef __HIP_DEVICE_COMPILE__
-    double cum = plane() < nm ? P->move_cum[plane() & (LDO_MAX_MOVES - 1)] : 0.0;
+    int mine = plane() & (LDO_MAX_MOVES - 1);
+    double cum = plane() < nm ? P->move_cum[mine] : 0.0;
+    mv_kind = P->move_kind[mine];
+    mv_maxreg = P->move_maxreg[mine];
+    track_range(P->L, mv_kind, mv_track, mv_width);
+    mv_att = 0;
+    mv_acc = 0;
 #endif
     for (int64_t n = 0; n < steps; n++) {
         if (S->status != ST_OK) {
@@ -2092,11 +2261,18 @@ DEVNI void WEng::simulate(int64_t steps) {
             m++;
         }
 #endif
-        S->attempts[m]++;
         bool acc = attempt(m);
-        if (acc) {
-            S->accepts[m]++;
+#ifdef __HIP_DEVICE_COMPILE__
+        bool own = plane() == m;
+        mv_att += own ? 1 : 0;
+        mv_acc += own & acc ? 1 : 0;
+        if ((n & 0x3FFFFFFF) == 0x3FFFFFFF) {
+            count_moves();
         }
+#else
+        S->attempts[m]++;
+        S->accepts[m] += acc ? 1 : 0;
+#endif
         track_move(m, acc);
         if (!acc) {
             reset_origami();
@@ -2114,6 +2290,9 @@ DEVNI void WEng::simulate(int64_t steps) {
             count_window_op();
         }
     }
+#ifdef __HIP_DEVICE_COMPILE__
+    count_moves();
+#endif
 }
 
 #undef S

@@ -473,8 +473,19 @@ DEV void net_layer1_lane(const Params& P, LearnedMove& m, int lane, int nl) {
     const float* e = W + P.net_off[1] + (int64_t)m.id * 16;
     for (int j = lane; j < 256; j += nl) {
         float s = W[P.net_off[3] + j];
-        for (int site = 0; site < 343; site++) {
-            s += W[P.net_off[0] + (int64_t)(site * 13 + m.ch[site]) * 256 + j];
+        const float* w1 = W + P.net_off[0] + j;
+        // 49 rows on their way at a time, added in site order
+#pragma unroll 1
+        for (int z = 0; z < 343; z += 49) {
+            float w[49];
+#pragma unroll
+            for (int q = 0; q < 49; q++) {
+                w[q] = w1[((z + q) * 13 + m.ch[z + q]) * 256];
+            }
+#pragma unroll
+            for (int q = 0; q < 49; q++) {
+                s += w[q];
+            }
         }
         for (int k = 0; k < 16; k++) {
             s = fmaf(e[k], W[P.net_off[2] + k * 256 + j], s);
@@ -489,8 +500,18 @@ DEV void net_dense_lane(const float* W, const float* b, const float* in, float* 
                         int n_out, bool relu, int lane, int nl) {
     for (int j = lane; j < n_out; j += nl) {
         float s = b[j];
-        for (int i = 0; i < n_in; i++) {
-            s = fmaf(in[i], W[(int64_t)i * n_out + j], s);
+        // 32 rows on their way at a time (n_in is a multiple of 32)
+#pragma unroll 1
+        for (int i0 = 0; i0 < n_in; i0 += 32) {
+            float w[32];
+#pragma unroll
+            for (int q = 0; q < 32; q++) {
+                w[q] = W[(i0 + q) * n_out + j];
+            }
+#pragma unroll
+            for (int q = 0; q < 32; q++) {
+                s = fmaf(in[i0 + q], w[q], s);
+            }
         }
         out[j] = relu ? fmaxf(s, 0.f) : s;
     }

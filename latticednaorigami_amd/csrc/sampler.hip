@@ -124,10 +124,13 @@ extern "C" __global__ void ldo_status_kernel(Params P, int32_t* out) {
 }
 
 // `attempts` learned domain-regrowth attempts per replica, one workgroup of
-// 64 lanes per replica: lane 0 runs the Markov chain, all lanes build the
-// input box and evaluate the network between barriers.  Each replica acts
-// with the control variables of its last sweep.
-extern "C" __global__ void __launch_bounds__(64)
+// 256 lanes per replica: lane 0 runs the Markov chain, all lanes build the
+// input box and evaluate the network between barriers, a hidden unit per lane
+// (with 64 lanes and four units each, an evaluation waited for four times as
+// many dependent rounds of weight loads).  Each replica acts with the control
+// variables of its last sweep.
+#define LDO_LEARNED_LANES 256
+extern "C" __global__ void __launch_bounds__(LDO_LEARNED_LANES)
     ldo_learned_kernel(Params P, int64_t attempts) {
     __shared__ Params sp;
     __shared__ Eng e;
@@ -156,7 +159,7 @@ extern "C" __global__ void __launch_bounds__(64)
         // regrowth one, an exchange one per growth path and placement)
         while (g == 1) {
             for (int ph = 0; ph < LDO_LEARNED_PHASES; ph++) {
-                learned_phase_lane(e, sp, m, ph, lane, 64);
+                learned_phase_lane(e, sp, m, ph, lane, LDO_LEARNED_LANES);
                 __syncthreads();
             }
             if (lane == 0) {
@@ -999,7 +1002,7 @@ int ldo_learned_sweep(void* ctx, int64_t attempts) {
         if (!c->P.net) {
             throw AbiError {LDO_E_MISUSE, "no network (ldo_learned_set_network)"};
         }
-        hipLaunchKernelGGL(ldo_learned_kernel, dim3(c->R), dim3(64), 0, c->stream, c->P,
+        hipLaunchKernelGGL(ldo_learned_kernel, dim3(c->R), dim3(LDO_LEARNED_LANES), 0, c->stream, c->P,
                            attempts);
         hip_check(hipGetLastError(), "launch learned");
         check_statuses(*c);

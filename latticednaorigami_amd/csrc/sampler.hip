@@ -86,12 +86,12 @@ extern "C" __global__ void ldo_sweep_kernel(Params P, int64_t steps, const int32
     }
 }
 
-extern "C" __global__ void ldo_dependent_kernel(Params P) {
-    bool active;
-    int r = replica_of_thread(P, active);
-    if (active) {
-        dependent_replica(P, r);
-    }
+// Dependent quantities of every replica, a wavefront each.
+extern "C" __global__ void __launch_bounds__(64) ldo_dependent_kernel(Params P) {
+    extern __shared__ int16_t chain_rank[]; // [nchain]
+#ifdef __HIP_DEVICE_COMPILE__
+    dependent_wave(P, blockIdx.x, chain_rank);
+#endif
 }
 
 extern "C" __global__ void ldo_exchange_kernel(Params P, XState X, int64_t swap_i,
@@ -289,16 +289,26 @@ extern "C" __global__ void ldo_batch_sweep_kernel(const Params* plist, int32_t n
     }
 }
 
-extern "C" __global__ void ldo_batch_scalars_kernel(const Params* plist, int32_t n,
-                                                    int32_t dependent, RepScalars* out) {
-    int k = blockIdx.x * blockDim.x + threadIdx.x;
+// Scalars of every chain, a wavefront each; with `dependent` its dependent
+// quantities first (LDS: 2 bytes per chain slot of the largest system).
+extern "C" __global__ void __launch_bounds__(64)
+    ldo_batch_scalars_kernel(const Params* plist, int32_t n, int32_t dependent, RepScalars* out) {
+    extern __shared__ int16_t chain_rank[];
+    int k = blockIdx.x;
     if (k >= n) {
         return;
     }
+    const Params& P = plist[k];
+#ifdef __HIP_DEVICE_COMPILE__
     if (dependent) {
-        dependent_replica(plist[k], 0);
+        dependent_wave(P, 0, chain_rank);
+        __syncthreads();
     }
-    out[k] = *(const RepScalars*)plist[k].blocks;
+#endif
+    const int32_t* src = (const int32_t*)P.blocks;
+    for (int i = threadIdx.x; i < (int)(sizeof(RepScalars) / 4); i += 64) {
+        ((int32_t*)(out + k))[i] = src[i];
+    }
 }
 
 // Staging of ldo_set_config_noalloc: the packed configuration (chain
@@ -1184,7 +1194,8 @@ int ldo_get_observables(void* ctx, int32_t replica, ldo_obs* out) {
         if (replica < 0 || replica >= c->R) {
             throw AbiError {LDO_E_ARG, "replica out of range"};
         }
-        hipLaunchKernelGGL(ldo_dependent_kernel, grid_of(*c), dim3(64), 0, c->stream, c->P);
+        hipLaunchKernelGGL(ldo_dependent_kernel, dim3(c->R), dim3(64),
+                           (size_t)c->P.L.nchain * sizeof(int16_t), c->stream, c->P);
         hip_check(hipGetLastError(), "launch dependent");
         RepScalars S;
         download(*c, &S, c->d_blocks + (size_t)replica * c->P.L.bytes, sizeof S, "copy scalars");
@@ -1413,8 +1424,13 @@ void free_batch(BatchCtx* b) {
 }
 
 void batch_scalars(BatchCtx& b, bool dependent, std::vector<RepScalars>& out) {
-    hipLaunchKernelGGL(ldo_batch_scalars_kernel, dim3((b.n + 63) / 64), dim3(64), 0, b.stream,
-                       b.d_params, b.n, (int32_t)dependent, b.d_scalars);
+    int32_t chains = 0;
+    for (const Params& P : b.params) {
+        chains = std::max(chains, P.L.nchain);
+    }
+    hipLaunchKernelGGL(ldo_batch_scalars_kernel, dim3(b.n), dim3(64),
+                       (size_t)chains * sizeof(int16_t), b.stream, b.d_params, b.n,
+                       (int32_t)dependent, b.d_scalars);
     hip_check(hipGetLastError(), "launch scalars");
     out.resize(b.n);
     bdownload(b, out.data(), b.d_scalars, (size_t)b.n * sizeof(RepScalars), "copy scalars");

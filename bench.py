@@ -39,7 +39,7 @@ N_CU = 256
 # a copy of known size; bench.py reads the measured HBM bytes per 1000-step
 # launch from the summary's "traffic_bytes_per_launch" line
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "ldo_sweep_lds_kernel_raster64_ptmc32_pmc.md")
-BATCH_TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "ldo_batch_sweep_kernel_batch4096.md")
+BATCH_TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "ldo_batch_sweep_lds_kernel_batch4096.md")
 MWUS3D_TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "ldo_sweep_lds_kernel_mwus3d.md")
 
 
@@ -202,7 +202,7 @@ def gpu_leg_batch(args):
     nbytes = algorithmic_bytes(c0, c1)
     achieved = nbytes / (kernel_ms / 1e3) / 1e9 if kernel_ms > 0 else None
     traffic = (profiled_traffic(BATCH_TRAFFIC_PROFILE)
-               if chosen == abi.BATCH_WAVE_SOLO and args.interval == 1000 else None)
+               if chosen == abi.BATCH_LDS and args.interval == 1000 else None)
     roofline = {
         "bound": "hbm",
         "achieved": achieved,

@@ -7,10 +7,10 @@
 //                        steps of GCMCSimulation::simulate; in PTMC mode it
 //                        first switches to its ladder slot (update_control_qs)
 //                        and ends with its dependent quantities
-//   ldo_sweep_lds_kernel the same sweep with the replica held in LDS: one
-//                        workgroup per replica copies its block, the launch
-//                        parameters and the engine object into LDS, runs the
-//                        chain there and writes the block back
+//   ldo_sweep_lds_kernel the same sweep on the wavefront engine
+//                        (engine_wave.h, sweep_wave.h): a wavefront copies its
+//                        replica's block into LDS, runs the chain there and
+//                        writes the block back
 //   ldo_exchange_kernel  one PTMC exchange round over even/odd ladder pairs
 //                        (OneDPTGCMCSimulation::attempt_exchange)
 // With lanes_per_replica = 64 every replica has a wavefront of its own, which
@@ -127,7 +127,8 @@ extern "C" __global__ void ldo_status_kernel(Params P, int32_t* out) {
 // 256 lanes per replica: lane 0 runs the Markov chain, all lanes build the
 // input box and evaluate the network between barriers, a hidden unit per lane
 // (with 64 lanes and four units each, an evaluation waited for four times as
-// many dependent rounds of weight loads).  Each replica acts with the control
+// many dependent rounds of weight loads: a round of 30 attempts and 100 steps
+// on 32 64-domain rasters took 9.3 ms and takes 7.4).  Each replica acts with the control
 // variables of its last sweep.
 #define LDO_LEARNED_LANES 256
 extern "C" __global__ void __launch_bounds__(LDO_LEARNED_LANES)
@@ -1444,9 +1445,9 @@ void batch_check(BatchCtx& b) {
     }
 }
 
-// Launches `steps` steps on every chain with the batch's sweep kernel and
-// returns the kernel time.
-// The groups of the LDS sweep (BatchCtx::groups).
+// The groups of the LDS sweep (BatchCtx::groups).  2048 chains of 8 to 128
+// domains, 500 steps: one launch 38.3 ms, groups 30.3 ms; 100 chains fit at
+// once, where a second launch only adds its overhead.
 void group_batch(BatchCtx& b) {
     std::vector<int32_t> order(b.n);
     std::vector<size_t> lds(b.n);
@@ -1481,6 +1482,8 @@ void group_batch(BatchCtx& b) {
     bupload(b, b.d_order, order, "copy order");
 }
 
+// Launches `steps` steps on every chain with the batch's sweep kernel and
+// returns the kernel time.
 double batch_launch(BatchCtx& b, int kernel, int64_t steps) {
     hip_check(hipEventRecord(b.ev0, b.stream), "event record");
     if (kernel == LDO_BATCH_LDS) {

@@ -334,17 +334,74 @@ DEV double exchange_uniform(const Params& P, int64_t rng_ctr, uint32_t& idx) {
     return (double)(x >> 11) * 0x1.0p-53;
 }
 
-// calc_acceptance_p + test_acceptance (ptmc_simulation.cpp:255-313) for the
-// replicas in slots a and b, swapping them when accepted.  The per-staple
+// One pair's attempt: its slots and replicas, the counter of its direction,
+// whether it may swap at all and the acceptance probability (1: without a
+// draw).  The pairs of a set share no slot, so what is read for one does not
+// depend on another's decision.
+struct PairTry {
+    int a, b, r1, r2;
+    size_t at; // counter offset
+    bool in;
+    double p;
+};
+
+DEV void exchange_swap(const Params& P, const XState& X, const PairTry& t) {
+    X.counts[2 + 2 * (size_t)P.n_replicas + t.at]++;
+    X.q_to_rep[t.a] = t.r2;
+    X.q_to_rep[t.b] = t.r1;
+    X.rep_slot[t.r2] = t.a;
+    X.rep_slot[t.r1] = t.b;
+}
+
+// test_acceptance (ptmc_simulation.cpp:300-313) and the swap
+DEV void exchange_decide(const Params& P, const XState& X, const PairTry& t, int64_t rng_ctr,
+                         uint32_t& idx) {
+    X.counts[0]++;
+    X.counts[2 + t.at]++;
+    if (t.in && ((t.p == 1) ? true : (t.p > exchange_uniform(P, rng_ctr, idx)))) {
+        X.counts[1]++;
+        exchange_swap(P, X, t);
+    }
+}
+
+#ifdef __HIP_DEVICE_COMPILE__
+// exchange_decide for the pairs of a wavefront's lanes (`active` ones, in lane
+// order) with Philox draws: a lane's draw is numbered by the drawing lanes
+// before it.
+__device__ __forceinline__ void exchange_decide_wave(const Params& P, const XState& X,
+                                                     const PairTry& t, bool active,
+                                                     int64_t rng_ctr, uint32_t& idx) {
+    int lane = threadIdx.x & 63;
+    bool draw = active && t.in && !(t.p == 1);
+    uint64_t m = __builtin_amdgcn_ballot_w64(draw);
+    bool accept = active && t.in;
+    if (draw) {
+        uint32_t k = idx + (uint32_t)__builtin_popcountll(m & ((1ull << lane) - 1));
+        accept = t.p > exchange_uniform(P, rng_ctr, k);
+    }
+    idx += (uint32_t)__builtin_popcountll(m);
+    uint64_t tried = __builtin_amdgcn_ballot_w64(active);
+    uint64_t taken = __builtin_amdgcn_ballot_w64(accept);
+    if (lane == 0) {
+        X.counts[0] += __builtin_popcountll(tried);
+        X.counts[1] += __builtin_popcountll(taken);
+    }
+    if (active) {
+        X.counts[2 + t.at]++;
+    }
+    if (accept) {
+        exchange_swap(P, X, t);
+    }
+}
+#endif
+
+// calc_acceptance_p (ptmc_simulation.cpp:255-298) for the replicas in slots a
+// and b.  The per-staple
 // chemical potential of a replica is reduced_u * T * (its own multiplier),
 // as update_staple_us leaves m_staple_us (origami_system.cpp:624-628).
 // d: direction of the pair (per-pair counters).
-DEV void exchange_pair(const Params& P, const XState& X, int a, int b, int d, int64_t rng_ctr,
-                       uint32_t& idx) {
-    int R = P.n_replicas;
+DEV PairTry exchange_pair(const Params& P, const XState& X, int a, int b, int d) {
     int nst = P.L.ntypes - 1;
-    X.counts[0]++;
-    X.counts[2 + (size_t)d * R + a]++;
     int r1 = X.q_to_rep[a], r2 = X.q_to_rep[b];
     RepScalars* S1 = (RepScalars*)(P.blocks + (size_t)r1 * P.L.bytes);
     RepScalars* S2 = (RepScalars*)(P.blocks + (size_t)r2 * P.L.bytes);
@@ -364,15 +421,7 @@ DEV void exchange_pair(const Params& P, const XState& X, int a, int b, int d, in
     double DBM = sm2 / t2 - sm1 / t1;
     double DBias = 0.0 * t2 - 0.0 * t1;
     double p = fmin(1.0, exp(DB * (DH + DBias) + DBM * Dst - dbu_dn));
-    bool accept = (p == 1) ? true : (p > exchange_uniform(P, rng_ctr, idx));
-    if (accept) {
-        X.counts[1]++;
-        X.counts[2 + 2 * (size_t)R + (size_t)d * R + a]++;
-        X.q_to_rep[a] = r2;
-        X.q_to_rep[b] = r1;
-        X.rep_slot[r2] = a;
-        X.rep_slot[r1] = b;
-    }
+    return PairTry {a, b, r1, r2, (size_t)d * P.n_replicas + a, true, p};
 }
 
 // One exchange round of the PT drivers: OneDPTGCMCSimulation::
@@ -397,13 +446,14 @@ DEV void exchange_round(const Params& P, const XState& X, int64_t swap_i, int64_
         for (int i = i0; i < i1; i += di) {
             for (int j = j0; j < j1; j += dj) {
                 int a = i * v2 + j;
-                exchange_pair(P, X, a, a + step, temps ? 0 : 1, rng_ctr, idx);
+                exchange_decide(P, X, exchange_pair(P, X, a, a + step, temps ? 0 : 1), rng_ctr,
+                                idx);
             }
         }
     }
     else {
         for (int i = (int)(swap_i % 2); i < R - 1; i += 2) {
-            exchange_pair(P, X, i, i + 1, 0, rng_ctr, idx);
+            exchange_decide(P, X, exchange_pair(P, X, i, i + 1, 0), rng_ctr, idx);
         }
     }
     int m = P.exchange_mode;
@@ -430,47 +480,28 @@ DEV double exchange_grid(const Params& P, int q, int p) {
 // adjacent windows swap configurations when each window's order parameter
 // lies inside the other window.  Windows are ladder slots here, so a swap
 // exchanges the two replicas' slots; each window keeps its stored biases.
-DEV void exchange_window_group(const Params& P, const XState& X, int64_t swap_i,
-                               int64_t rng_ctr, int g0, int g1, uint32_t& idx) {
-    for (int i = g0 + (int)(swap_i % 2); i < g1 - 1; i += 2) {
-        X.counts[0]++;
-        X.counts[2 + i]++;
-        const ldo_window& w1 = P.windows[i];
-        const ldo_window& w2 = P.windows[i + 1];
-        int r1 = X.q_to_rep[i], r2 = X.q_to_rep[i + 1];
-        int p1 = replica_window_op(P, r1, w1);
-        int p2 = replica_window_op(P, r2, w2);
-        if (p2 < w1.min_op || p2 > w1.max_op || p1 < w2.min_op || p1 > w2.max_op) {
-            continue;
-        }
-        bool accept = true;
-        if (p1 != p2) {
-            double d1 = exchange_grid(P, i, p1) - exchange_grid(P, i + 1, p1);
-            double d2 = exchange_grid(P, i + 1, p2) - exchange_grid(P, i, p2);
-            double p = fmin(1.0, exp(d1 + d2));
-            accept = (p == 1) ? true : (p > exchange_uniform(P, rng_ctr, idx));
-        }
-        if (accept) {
-            X.counts[1]++;
-            X.counts[2 + 2 * (size_t)P.n_replicas + i]++;
-            X.q_to_rep[i] = r2;
-            X.q_to_rep[i + 1] = r1;
-            X.rep_slot[r2] = i;
-            X.rep_slot[r1] = i + 1;
-        }
+DEV PairTry exchange_window_pair(const Params& P, const XState& X, int i) {
+    const ldo_window& w1 = P.windows[i];
+    const ldo_window& w2 = P.windows[i + 1];
+    int r1 = X.q_to_rep[i], r2 = X.q_to_rep[i + 1];
+    int p1 = replica_window_op(P, r1, w1);
+    int p2 = replica_window_op(P, r2, w2);
+    bool in = !(p2 < w1.min_op || p2 > w1.max_op || p1 < w2.min_op || p1 > w2.max_op);
+    double p = 1;
+    if (in && p1 != p2) {
+        double d1 = exchange_grid(P, i, p1) - exchange_grid(P, i + 1, p1);
+        double d2 = exchange_grid(P, i + 1, p2) - exchange_grid(P, i, p2);
+        p = fmin(1.0, exp(d1 + d2));
     }
+    return PairTry {i, i + 1, r1, r2, (size_t)i, in, p};
 }
 
 // Swap of the replicas in window w of two ladders at neighbouring
 // temperatures (slots a < b, LDO_FLAG_WINDOW_TEMPERATURE_SWAPS): the PTMC log
 // ratio of the two slots plus the grid biases of both windows at both
 // replicas' order parameters; the windows' restraints are equal and cancel.
-DEV void exchange_window_temperatures(const Params& P, const XState& X, int a, int b,
-                                      int64_t rng_ctr, uint32_t& idx) {
-    int R = P.n_replicas;
+DEV PairTry exchange_window_temperatures(const Params& P, const XState& X, int a, int b) {
     int nst = P.L.ntypes - 1;
-    X.counts[0]++;
-    X.counts[2 + (size_t)R + a]++;
     int r1 = X.q_to_rep[a], r2 = X.q_to_rep[b];
     const RepScalars* S1 = (const RepScalars*)(P.blocks + (size_t)r1 * P.L.bytes);
     const RepScalars* S2 = (const RepScalars*)(P.blocks + (size_t)r2 * P.L.bytes);
@@ -493,15 +524,7 @@ DEV void exchange_window_temperatures(const Params& P, const XState& X, int a, i
     double dg = (exchange_grid(P, a, p1) - exchange_grid(P, b, p1)) +
                 (exchange_grid(P, b, p2) - exchange_grid(P, a, p2));
     double p = fmin(1.0, exp(DB * DH + DBM * Dst - dbu_dn + P.windows[a].bias_mult * dg));
-    bool accept = (p == 1) ? true : (p > exchange_uniform(P, rng_ctr, idx));
-    if (accept) {
-        X.counts[1]++;
-        X.counts[2 + 3 * (size_t)R + a]++;
-        X.q_to_rep[a] = r2;
-        X.q_to_rep[b] = r1;
-        X.rep_slot[r2] = a;
-        X.rep_slot[r1] = b;
-    }
+    return PairTry {a, b, r1, r2, (size_t)P.n_replicas + a, true, p};
 }
 
 // One exchange round over every window ladder.
@@ -518,16 +541,98 @@ DEV void exchange_windows_round(const Params& P, const XState& X, int64_t swap_i
         if (g0 == 0) {
             W = g1;
         }
-        exchange_window_group(P, X, swap_i, rng_ctr, g0, g1, idx);
+        for (int i = g0 + (int)(swap_i % 2); i < g1 - 1; i += 2) {
+            exchange_decide(P, X, exchange_window_pair(P, X, i), rng_ctr, idx);
+        }
     }
     if (P.flags & LDO_FLAG_WINDOW_TEMPERATURE_SWAPS) {
         for (int g = (int)(swap_i % 2); (g + 2) * W <= R; g += 2) {
             for (int w = 0; w < W; w++) {
-                exchange_window_temperatures(P, X, g * W + w, (g + 1) * W + w, rng_ctr, idx);
+                exchange_decide(P, X,
+                                exchange_window_temperatures(P, X, g * W + w, (g + 1) * W + w),
+                                rng_ctr, idx);
             }
         }
     }
 }
+
+#ifdef __HIP_DEVICE_COMPILE__
+// Both rounds by a wavefront, for Philox draws: a pair per lane, the pairs of
+// a set 64 at a time in the order above.  A pair reads some hundred values in
+// dependent rounds (a staple type at a time), which is all an exchange takes:
+// one lane needed 1.4 ms for the 192 pairs of 256 windows.
+__device__ __forceinline__ void exchange_round_wave(const Params& P, const XState& X,
+                                                    int64_t swap_i, int64_t rng_ctr) {
+    int R = P.n_replicas, lane = threadIdx.x & 63;
+    uint32_t idx = 0;
+    bool grid = P.exchange_mode == LDO_EXCHANGE_2D;
+    int v2 = grid ? P.pt_dim2 : 1, set = (int)(swap_i % 4);
+    bool temps = !grid || set % 2 == 0;
+    // pairs (i, j) of the grid from (i0, j0) in steps (di, dj), nj to a row
+    int i0 = grid ? set == 2 : (int)(swap_i % 2), j0 = grid && set == 3 ? 1 : 0;
+    int di = temps ? 2 : 1, dj = !grid || temps ? 1 : 2;
+    int i1 = grid && !temps ? R / v2 : R / v2 - 1, j1 = temps ? v2 : v2 - 1;
+    int ni = i1 > i0 ? (i1 - i0 + di - 1) / di : 0, nj = j1 > j0 ? (j1 - j0 + dj - 1) / dj : 0;
+    int step = temps ? v2 : 1;
+    for (int k0 = 0; k0 < ni * nj; k0 += 64) {
+        int k = k0 + lane;
+        bool active = k < ni * nj;
+        PairTry t = {};
+        if (active) {
+            int a = (i0 + di * (k / nj)) * v2 + j0 + dj * (k % nj);
+            t = exchange_pair(P, X, a, a + step, temps ? 0 : 1);
+        }
+        exchange_decide_wave(P, X, t, active, rng_ctr, idx);
+    }
+    __syncthreads();
+    int m = P.exchange_mode;
+    if (m == LDO_EXCHANGE_TEMPERATURE || m == LDO_EXCHANGE_HUT || m == LDO_EXCHANGE_2D) {
+        for (int q = lane; q < R; q += 64) {
+            X.rep_u[X.q_to_rep[q]] = X.ladder_u[q];
+        }
+    }
+}
+
+__device__ __forceinline__ void exchange_windows_round_wave(const Params& P, const XState& X,
+                                                            int64_t swap_i, int64_t rng_ctr) {
+    int R = P.n_replicas, lane = threadIdx.x & 63;
+    uint32_t idx = 0;
+    int W = R, g0 = 0; // the first ladder's windows; start of the current one
+    for (int k0 = 0; k0 < R; k0 += 64) {
+        int i = k0 + lane;
+        bool first = i < R && i > 0 && X.ladder_t[i] != X.ladder_t[i - 1];
+        uint64_t m = __builtin_amdgcn_ballot_w64(first);
+        uint64_t below = m & (~0ull >> (63 - lane));
+        int g = below ? k0 + 63 - __builtin_clzll(below) : g0;
+        bool active = i < R - 1 && X.ladder_t[i + 1] == X.ladder_t[i] &&
+                      (i - g) % 2 == (int)(swap_i % 2);
+        PairTry t = {};
+        if (active) {
+            t = exchange_window_pair(P, X, i);
+        }
+        exchange_decide_wave(P, X, t, active, rng_ctr, idx);
+        if (m) {
+            W = W == R ? k0 + __builtin_ctzll(m) : W;
+            g0 = k0 + 63 - __builtin_clzll(m);
+        }
+    }
+    __syncthreads();
+    if (P.flags & LDO_FLAG_WINDOW_TEMPERATURE_SWAPS) {
+        // ladder pairs (g, g + 1), W windows each
+        int s = (int)(swap_i % 2), n = R / W - s;
+        n = n > 0 ? n / 2 * W : 0;
+        for (int k0 = 0; k0 < n; k0 += 64) {
+            int k = k0 + lane;
+            PairTry t = {};
+            if (k < n) {
+                int a = (s + 2 * (k / W)) * W + k % W;
+                t = exchange_window_temperatures(P, X, a, a + W);
+            }
+            exchange_decide_wave(P, X, t, k < n, rng_ctr, idx);
+        }
+    }
+}
+#endif
 
 // the stored move-level bias of the window in ladder slot q (0 without
 // windows).  The replica in slot q is rep_slot's inverse, not the block's

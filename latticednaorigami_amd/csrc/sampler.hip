@@ -94,8 +94,20 @@ extern "C" __global__ void __launch_bounds__(64) ldo_dependent_kernel(Params P) 
 #endif
 }
 
-extern "C" __global__ void ldo_exchange_kernel(Params P, XState X, int64_t swap_i,
+extern "C" __global__ void __launch_bounds__(64) ldo_exchange_kernel(Params P, XState X, int64_t swap_i,
                                                int64_t rng_ctr) {
+#ifdef __HIP_DEVICE_COMPILE__
+    // a wavefront; recorded draws are taken one by one
+    if (P.rng_mode != 1) {
+        if (P.exchange_mode == LDO_EXCHANGE_WINDOWS) {
+            exchange_windows_round_wave(P, X, swap_i, rng_ctr);
+        }
+        else {
+            exchange_round_wave(P, X, swap_i, rng_ctr);
+        }
+        return;
+    }
+#endif
     if (threadIdx.x == 0 && blockIdx.x == 0) {
         if (P.exchange_mode == LDO_EXCHANGE_WINDOWS) {
             exchange_windows_round(P, X, swap_i, rng_ctr);

@@ -7,6 +7,7 @@ run on that build: they check the engine's logic step for step against the
 oracle wherever no GPU is at hand.
 """
 import ctypes as C
+import fcntl
 import os
 import subprocess
 
@@ -45,14 +46,28 @@ class HostLib:
 
 @pytest.fixture(scope="module")
 def sampler_cls():
-    # make knows the sources the library depends on; a failed build fails the tests
-    subprocess.run(["make", "-C", HOST_DIR], check=True, capture_output=True)
+    # make knows the sources the library depends on; a failed build fails the
+    # tests, and test processes side by side build one after the other
+    lock = os.open(HOST_DIR, os.O_RDONLY)
+    try:
+        fcntl.flock(lock, fcntl.LOCK_EX)
+        subprocess.run(["make", "-C", HOST_DIR], check=True, capture_output=True)
+    finally:
+        os.close(lock)
     lib = HostLib(C.CDLL(HOST_LIB))
     from latticednaorigami_amd.sampler import Sampler
 
     def make(system, **kw):
         return Sampler(system, lib=lib, **kw)
     return make
+
+
+@pytest.fixture(autouse=True, params=["wave", "general"])
+def engine(request, monkeypatch):
+    """Every case on the wavefront engine, which sweeps blocks that fit LDS, and on the
+    general engine, which sweeps the others and those of one lane per replica."""
+    if request.param == "general":
+        monkeypatch.setenv("LDO_SWEEP_KERNEL", "global")
 
 
 def test_host_build_is_current(sampler_cls):

@@ -162,6 +162,10 @@ int guarded(HostCtx* c, F f) {
 
 extern "C" {
 
+// the site hash's home index, for the test of its spread
+int eh_site_home(int32_t x, int32_t y, int32_t z, int32_t bits) { return site_home(x, y, z, bits); }
+
+
 int eh_create(const ldo_system_desc* sys, const ldo_run_params* run, const ldo_config* init,
               int32_t n_replicas, const double* temps, void** out_ctx) {
     HostCtx* c = new HostCtx;

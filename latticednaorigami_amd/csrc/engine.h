@@ -66,6 +66,45 @@ DEV int unit_index(I3 v) {
     return v.z > 0 ? 4 : 5;
 }
 
+// VectorThree::rotate_half (utility.cpp:68-85)
+DEV I3 rotate_half3(I3 v, I3 axis) {
+    int ax = axis.x < 0 ? -axis.x : axis.x;
+    int ay = axis.y < 0 ? -axis.y : axis.y;
+    int az = axis.z < 0 ? -axis.z : axis.z;
+    if (ax == 1 && ay == 0 && az == 0) {
+        return i3(v.x, -v.y, -v.z);
+    }
+    if (ax == 0 && ay == 1 && az == 0) {
+        return i3(-v.x, v.y, -v.z);
+    }
+    if (ax == 0 && ay == 0 && az == 1) {
+        return i3(-v.x, -v.y, v.z);
+    }
+    return v;
+}
+
+// VectorThree::rotate(axis, -1) (utility.cpp:102-142): the quarter turn the
+// ThreeQuarterTurn twist rule uses.
+DEV I3 rotate_minus_quarter3(I3 v, I3 axis) {
+    int dir = -1;
+    int ax = axis.x < 0 ? -axis.x : axis.x;
+    int ay = axis.y < 0 ? -axis.y : axis.y;
+    int az = axis.z < 0 ? -axis.z : axis.z;
+    if (axis.x != ax || axis.y != ay || axis.z != az) {
+        dir = -dir;
+    }
+    if (ax == 1 && ay == 0 && az == 0) {
+        return i3(v.x, -dir * v.z, dir * v.y);
+    }
+    if (ax == 0 && ay == 1 && az == 0) {
+        return i3(-dir * v.z, v.y, dir * v.x);
+    }
+    if (ax == 0 && ay == 0 && az == 1) {
+        return i3(-dir * v.y, dir * v.x, v.z);
+    }
+    return v;
+}
+
 struct Delta {
     double e;
     int st;
@@ -524,7 +563,93 @@ struct Eng {
         hash[i] = LDO_HASH_EMPTY;
     }
 
+    // ------------------------------------------------------------ rules
+    // HalfTurnDomain / ThreeQuarterTurnDomain::check_twist_constraint
+    // (domain.cpp:33-40, 69-78)
+    DEV bool twist_ok(int a, I3 ndr, int b) const {
+        I3 r = (dtype == 0) ? rotate_half3(ore(a), ndr)
+                                     : rotate_minus_quarter3(ore(a), ndr);
+        return eq3(r, ore(b));
+    }
+    // check_kink_constraint (domain.cpp:42-57, 80-97)
+    DEV bool kink_ok(int a, I3 ndr, int b) const {
+        I3 oa = ore(a), ob = ore(b);
+        if (eq3(ndr, neg3(oa))) {
+            return false;
+        }
+        if (eq3(ndr, oa)) {
+            if (dtype == 0) {
+                return !eq3(ob, neg3(oa));
+            }
+            return !(eq3(oa, ob) || eq3(oa, neg3(ob)));
+        }
+        if (eq3(ndr, ob) || eq3(ndr, neg3(ob))) {
+            return false;
+        }
+        return true;
+    }
+    // check_junction_constraint (domain.cpp:59-67, 99-118)
+    DEV bool junction_ok(int j1, int j2, int k1, int k2) const {
+        if (dtype == 0) {
+            return true;
+        }
+        I3 nk = sub3(pos(k2), pos(k1));
+        if (eq3(nk, ore(k1))) {
+            I3 n1 = sub3(pos(j2), pos(j1));
+            if (d_of(j1) > d_of(j2)) {
+                n1 = neg3(n1);
+            }
+            if (!twist_ok(k1, n1, k2)) {
+                return false;
+            }
+        }
+        return true;
+    }
+    // doubly_contiguous (origami_potential.cpp:51-68)
+    DEV bool doubly_contig(int a, int b) const {
+        if (cslot_of(a) != cslot_of(b) || d_of(b) != d_of(a) + 1) {
+            return false;
+        }
+        int ba = bd(a), bb = bd(b);
+        if (cslot_of(ba) != cslot_of(bb)) {
+            return false;
+        }
+        int dd = d_of(bb) - d_of(ba);
+        return dd == 1 || dd == -1;
+    }
+    // check_pair_stacked (origami_potential.cpp:70-83)
+    DEV bool pair_stacked(int a, int b) const {
+        if (d_of(a) > d_of(b)) {
+            int t = a;
+            a = b;
+            b = t;
+        }
+        I3 ndr = sub3(pos(b), pos(a));
+        I3 oa = ore(a);
+        if (!eq3(ndr, oa) && !eq3(ndr, neg3(oa))) {
+            return twist_ok(a, ndr, b);
+        }
+        return false;
+    }
+
     // ------------------------------------------------------------ FourBody
+    DEVIN void fb_single(int h1, int h2, int h3);
+    DEVIN void fb_double(int h1, int h2, int h3);
+    DEVIN void fb_triply(int h1, int h2, int h3);
+    DEVNI void fb_junction(int j1, int j2, int j3, int j4, int k1, int k2);
+    DEVIN void fb_junction_pair(int a, int b, int j);
+    DEVIN void fb_backward_triplets(int a, int b);
+    DEVIN void fb_forward_triplets(int a, int b);
+    DEVIN void fb_central_triplets(int di, int dj);
+    DEVIN void fb_backward_single_junction(int a, int b);
+    DEVIN void fb_backward_outer(int j3, int j4, int k2, int k1);
+    DEVIN void fb_forward_outer(int j1, int j2, int k1, int k2);
+    DEVIN void fb_central_outer(int j1, int j2, int k1, int k2, int k2b);
+    DEVIN void fb_forward_single_junction(int a, int b);
+    DEVIN void fb_central_single_junction(int a, int b);
+    DEVIN void fb_regular_pair(int a, int b, int i);
+    DEVIN void fb_helix_pair(int a, int b, int i, int j);
+    DEVIN void fb_around(int cd, int j);
     DEVNI void fb_terms(int di, int dj);
     DEVIN Delta bind_domain(int di);
 

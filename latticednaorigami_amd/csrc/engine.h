@@ -488,25 +488,43 @@ struct Eng {
     // ------------------------------------------------------------ site hash
     // the 16-bit home index of a site (layout.h)
     DEV int home(I3 p) const { return site_home(p.x, p.y, p.z, hbits); }
-    // index of site p's entry, -1 for an empty site
-    DEV int hfind(I3 p) const {
+    // a slot's record in one read: position and packed word
+    struct DomWords {
+        int32_t x, y, z;
+        uint32_t w;
+    };
+    DEV DomWords words(int s) const {
+        DomWords r;
+        __builtin_memcpy(&r, __builtin_assume_aligned(dom + s, 16), sizeof r);
+        return r;
+    }
+    // index of site p's entry, -1 for an empty site; w: its record's packed word
+    DEV int hfind(I3 p, uint32_t& w) const {
         int h = home(p), i = h;
         for (int n = 0; n <= hmask; n++) {
             uint32_t v = hash[i];
             if (v == LDO_HASH_EMPTY) {
                 return -1;
             }
-            if ((int)(v >> 16) == h && eq3(pos((int)(v & 0xFFFFu)), p)) {
-                return i;
+            if ((int)(v >> 16) == h) {
+                DomWords r = words((int)(v & 0xFFFFu));
+                if (r.x == p.x && r.y == p.y && r.z == p.z) {
+                    w = r.w;
+                    return i;
+                }
             }
             i = (i + 1) & hmask;
         }
         return -1;
     }
+    DEV int hfind(I3 p) const {
+        uint32_t w;
+        return hfind(p, w);
+    }
     // OrigamiSystem::position_occupancy (origami_system.cpp:193-202)
     DEV int occupancy(I3 p) {
-        int i = hfind(p);
-        return i < 0 ? OCC_UNASSIGNED : (int)dom[hash[i] & 0xFFFFu].state;
+        uint32_t w = 0;
+        return hfind(p, w) < 0 ? OCC_UNASSIGNED : (int)((w >> 8) & 0xFFu);
     }
     DEV int unbound_at(I3 p) {
         int i = hfind(p);

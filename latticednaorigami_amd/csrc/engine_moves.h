@@ -345,10 +345,11 @@ DEVNI void LDO_ENG::cb_select_and_set(int d, int prev_d) {
     bool looked = par && dom[d].state == OCC_UNASSIGNED;
     int occ_l = OCC_UNASSIGNED, ub_l = -1;
     if (looked && plane() < 6) {
-        int hi = hfind(add3(pp, unit3(plane())));
+        uint32_t w = 0;
+        int hi = hfind(add3(pp, unit3(plane())), w);
         if (hi >= 0) {
             ub_l = (int)(hash[hi] & 0xFFFFu);
-            occ_l = dom[ub_l].state;
+            occ_l = (int)((w >> 8) & 0xFFu);
         }
     }
 #pragma unroll

@@ -157,7 +157,7 @@ typedef struct ldo_run_params {
     uint64_t seed;
     int32_t rng_mode;      /* ldo_rng_mode */
     int32_t exchange_mode; /* ldo_exchange_mode */
-    int32_t lanes_per_replica; /* 0: pick automatically; 1 or 64 */
+    int32_t lanes_per_replica; /* 0: by replica count and block size; 1 or 64 */
     int32_t flags;             /* ldo_run_flags, 0 = the reference's behaviour */
     /* CTRG recoil growth (simulation.cpp:493-495): max_num_recoils (>= 0) and
      * max_c_attempts (1..36) per movetype; read for CTRG entries only, and

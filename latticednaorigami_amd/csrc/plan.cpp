@@ -285,7 +285,7 @@ void make_plan(const ldo_system_desc* sys, const ldo_run_params* run, int32_t n_
     P.fugacity = sys->staple_M;
     int lpr = run->lanes_per_replica;
     if (lpr == 0) {
-        lpr = n_replicas >= 2048 ? 1 : 64;
+        lpr = 64; // until it is known whether the block fits LDS (default_lanes)
     }
     if (lpr != 1 && lpr != 64) {
         throw AbiError {LDO_E_ARG, "lanes_per_replica must be 0, 1 or 64"};
@@ -329,6 +329,10 @@ void make_plan(const ldo_system_desc* sys, const ldo_run_params* run, int32_t n_
             out.reduced_u[(size_t)r * nst + t] = u / temps[r];
         }
     }
+}
+
+int default_lanes(int n_replicas, bool lds) {
+    return !lds && n_replicas > 40000 ? 1 : 64;
 }
 
 void slot_tables(const Plan& p, std::vector<double>& tab, std::vector<double>& init) {

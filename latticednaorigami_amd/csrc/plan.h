@@ -61,6 +61,14 @@ std::vector<double> ladder_values(const Plan& p);
 // Modes without a ladder keep the slot's value.
 double slot_stacking(const Plan& p, int q);
 
+// Lanes per replica where the caller leaves the choice (lanes_per_replica = 0);
+// lds: the replicas' blocks fit LDS.  There a wavefront per replica is always
+// the faster form: 50 steps of 2048, 16 384 and 65 536 four-domain replicas take
+// 1.8, 9.5 and 35 ms, with a lane each 92, 96 and 136.  In device memory a
+// wavefront each takes 9.5 and 92 ms at 2048 and 32 768 replicas, a lane each 92
+// and 105; at 49 152 it is 135 and 119, at 65 536 179 and 136.
+int default_lanes(int n_replicas, bool lds);
+
 // Table key class of every slot: slots with the same (temperature, sweep
 // stacking multiplier) share a class, numbered from 0 in order of first
 // appearance.  A table-cache hit keeps the initiation terms of the last

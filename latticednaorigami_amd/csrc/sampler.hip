@@ -788,6 +788,9 @@ int ldo_create(const ldo_system_desc* sys, const ldo_run_params* run, const ldo_
         hip_check(hipGetLastError(), "launch init");
         check_statuses(*c);
         choose_sweep_kernel(*c);
+        if (run->lanes_per_replica == 0) {
+            P.lanes_per_replica = ldo::default_lanes(n_replicas, c->lds_sweep);
+        }
     });
     if (rc != LDO_OK) {
         free_ctx(c);

@@ -29,6 +29,7 @@ struct HostCtx {
     ldo::Plan plan;
     Params P {};
     int R = 0;
+    bool general = false; // LDO_SWEEP_KERNEL=global at creation, as in the library
     int64_t swap_counter = 0;
     int64_t swap_base = 0;
     std::string err;
@@ -75,9 +76,7 @@ void learned_replica(const Params& P, int r, int64_t attempts) {
 // a staged copy of the block with a wavefront per replica, else (or with
 // LDO_SWEEP_KERNEL=global) the general engine on the block itself.
 void sweep_one(const HostCtx& c, int r, int64_t steps, const int32_t* rep_slot) {
-    const char* force = std::getenv("LDO_SWEEP_KERNEL");
-    bool global = force != nullptr && std::strcmp(force, "global") == 0;
-    if (global || c.P.lanes_per_replica != 64) {
+    if (c.general || c.P.lanes_per_replica != 64) {
         sweep_replica(c.P, r, steps, rep_slot);
         return;
     }
@@ -162,6 +161,11 @@ int guarded(HostCtx* c, F f) {
 
 extern "C" {
 
+// lanes per replica where the caller leaves the choice
+int eh_default_lanes(int32_t n_replicas, int32_t lds) {
+    return ldo::default_lanes(n_replicas, lds != 0);
+}
+
 // the site hash's home index, for the test of its spread
 int eh_site_home(int32_t x, int32_t y, int32_t z, int32_t bits) { return site_home(x, y, z, bits); }
 
@@ -176,6 +180,8 @@ int eh_create(const ldo_system_desc* sys, const ldo_run_params* run, const ldo_c
         ldo::make_plan(sys, run, n_replicas, temps, c->plan);
         c->P = c->plan.P;
         c->R = n_replicas;
+        const char* force = std::getenv("LDO_SWEEP_KERNEL");
+        c->general = force != nullptr && std::strcmp(force, "global") == 0;
         c->P.type_len = c->plan.type_len.data();
         c->P.type_ident = c->plan.type_ident.data();
         set_tables(*c);

@@ -5,13 +5,15 @@ misbinding, more staples than a wavefront has lanes, staples of up to eight
 domains in strides with unused slots, and centring and constraint checks every
 few steps.  Each runs step for step against the CPU oracle, on the host build
 of the engine and on the GPU, and the general engine runs beside it."""
+import ctypes as C
 import dataclasses
 import os
+import time
 
 import pytest
 
 import parity_cases as pc
-from test_engine_host_parity import sampler_cls as host_sampler  # noqa: F401
+from test_engine_host_parity import HOST_LIB, sampler_cls as host_sampler  # noqa: F401
 from latticednaorigami_amd import abi, systems
 
 RING = [(0, 0, 0), (1, 0, 0), (2, 0, 0), (3, 0, 0), (3, 1, 0), (2, 1, 0), (1, 1, 0), (0, 1, 0)]
@@ -98,6 +100,36 @@ def test_forms_on_the_host_build(host_sampler, oracle_mod, name):  # noqa: F811
     wave = check(host_sampler, oracle_mod, name)
     if name == "crowded":
         assert max(wave.observables(r)["num_staples"] for r in range(2)) > 64
+
+
+def test_default_lanes(host_sampler):  # noqa: F811
+    """A wavefront per replica for every count where the block fits LDS, and up to
+    40 000 where it does not."""
+    lanes = C.CDLL(HOST_LIB).eh_default_lanes
+    for n in (1, 2047, 2048, 40000, 40001, 65536):
+        assert lanes(n, 1) == 64
+        assert lanes(n, 0) == (64 if n <= 40000 else 1)
+
+
+@pytest.mark.gpu
+def test_replica_counts_around_2048_run_alike():
+    """2048 replicas take the kernel that 2047 take: the same chains in about the same
+    time (a lane per replica, the default there before, took 50 times as long)."""
+    from latticednaorigami_amd.sampler import Sampler
+    s = systems.four_domain_system(max_total_staples=8)
+    temps = [320.0 + 0.01 * i for i in range(2048)]
+    times, obs = {}, {}
+    for n in (2047, 2048):
+        print("replicas", n, flush=True)
+        x = Sampler(s, temps=temps[:n])
+        x.sweep(100)
+        t0 = time.perf_counter()
+        x.sweep(100)
+        times[n] = time.perf_counter() - t0
+        obs[n] = [x.observables(r) for r in (0, 1000, 2046)]
+        x.close()
+    assert obs[2047] == obs[2048]
+    assert times[2048] < 10 * times[2047]
 
 
 @pytest.mark.gpu

@@ -256,9 +256,6 @@ struct Eng {
     // stores.  Sections start 16-byte aligned and own the padding up to the
     // next 16-byte boundary (the replica-block layout rounds every section).
     DEV void fill_section(void* base, int64_t bytes, uint32_t pattern) {
-        struct alignas(16) Quad {
-            uint32_t a, b, c, d;
-        };
         Quad q {pattern, pattern, pattern, pattern};
         Quad* dst = (Quad*)base;
         for (int64_t i = plane(), n = (bytes + 15) / 16; i < n; i += pwidth()) {

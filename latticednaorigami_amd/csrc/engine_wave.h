@@ -125,7 +125,7 @@ struct LPosOre {
     LRef<int32_t> x, y, z, ore;
     DEV explicit LPosOre(lds_t q) : p(q), x {q}, y {q + 4}, z {q + 8}, ore {q + 12} {}
     DEV void operator=(const LPosOre& o) const {
-        *(LDO_LDS uint4*)p = *(LDO_LDS const uint4*)o.p;
+        *(LDO_LDS Quad*)p = *(LDO_LDS const Quad*)o.p;
     }
 };
 struct LChain {
@@ -193,7 +193,7 @@ struct FbLds {
     int stack_one;
     int ns, lmask, cyc, dtype, n_ident;
     DEV FbRec rec(int s) const {
-        uint4 v = *(LDO_LDS const uint4*)(dom + s * 16);
+        Quad v = *(LDO_LDS const Quad*)(dom + s * 16);
         return FbRec {uni((int32_t)v.x), uni((int32_t)v.y), uni((int32_t)v.z), uni(v.w)};
     }
     DEV double stk(int p, int q) const {
@@ -216,7 +216,7 @@ struct FbLane {
     lds_t dom;
     int ns, lmask, cyc, dtype;
     DEV FbRec rec(int s) const {
-        uint4 v = *(LDO_LDS const uint4*)(dom + s * 16);
+        Quad v = *(LDO_LDS const Quad*)(dom + s * 16);
         return FbRec {(int32_t)v.x, (int32_t)v.y, (int32_t)v.z, v.w};
     }
     DEV double stk(int, int) const { return 0; }
@@ -467,9 +467,9 @@ struct WEng {
 
     template <class T>
     DEV void fill_section(LArr<T> a, int64_t bytes, uint32_t pattern) {
-        uint4 q = make_uint4(pattern, pattern, pattern, pattern);
+        Quad q {pattern, pattern, pattern, pattern};
         for (int i = plane(), n = (int)((bytes + 15) / 16); i < n; i += width) {
-            *(LDO_LDS uint4*)(a.p + 16 * i) = q;
+            *(LDO_LDS Quad*)(a.p + 16 * i) = q;
         }
     }
 
@@ -731,12 +731,12 @@ struct WEng {
 
     // a domain's record in one read
     DEV FbRec rec(int s) const {
-        uint4 v = *(LDO_LDS const uint4*)(dom.p + s * 16);
+        Quad v = *(LDO_LDS const Quad*)(dom.p + s * 16);
         return FbRec {uni((int32_t)v.x), uni((int32_t)v.y), uni((int32_t)v.z), uni(v.w)};
     }
     DEV void put_rec(int s, I3 p, uint32_t w) const {
-        *(LDO_LDS uint4*)(dom.p + s * 16) =
-            make_uint4((uint32_t)p.x, (uint32_t)p.y, (uint32_t)p.z, w);
+        *(LDO_LDS Quad*)(dom.p + s * 16) =
+            Quad {(uint32_t)p.x, (uint32_t)p.y, (uint32_t)p.z, w};
     }
     static DEV uint32_t pack(int ore, int state, int bound) {
         return (uint32_t)ore | (uint32_t)state << 8 | (uint32_t)(uint16_t)bound << 16;
@@ -753,9 +753,9 @@ struct WEng {
     DEV int ident_of(int s) const { return dident[s] + ident_lo; }
     // prev[s] = the domain's position and orientation
     DEV void save_prev(int s) const {
-        uint4 v = *(LDO_LDS const uint4*)(dom.p + s * 16);
+        Quad v = *(LDO_LDS const Quad*)(dom.p + s * 16);
         v.w &= 0xFFu;
-        *(LDO_LDS uint4*)(prev.p + s * 16) = v;
+        *(LDO_LDS Quad*)(prev.p + s * 16) = v;
     }
     // binding energy of s and t; `comp`: their identities are complementary
     DEV double hyb(int s, int t, bool comp) const {
@@ -1600,7 +1600,7 @@ __device__ __forceinline__ void WEng::look_six(int d, I3 pp) {
     uint32_t gfree = (uint32_t)(ballot(en == LDO_HASH_EMPTY) >> (lane & 56)) & 255u;
     bool cand = site & ((int)(en >> 16) == six_h) & ((gfree & ((1u << j) - 1)) == 0);
     int s = cand ? (int)(en & 0xFFFFu) : 0;
-    uint4 r = *(LDO_LDS const uint4*)(dom.p + s * 16);
+    Quad r = *(LDO_LDS const Quad*)(dom.p + s * 16);
     bool hit = cand & ((int)r.x == six_p.x) & ((int)r.y == six_p.y) & ((int)r.z == six_p.z);
     uint32_t ghit = (uint32_t)(ballot(hit) >> (lane & 56)) & 255u;
     int src = ((lane & 56) | __builtin_ctz(ghit | 256u)) << 2;
@@ -1652,7 +1652,7 @@ __device__ __forceinline__ void WEng::walk_six(int d, int sg, int std_) {
         uint32_t k = 0xFFFFu;
         int es = -1, ex = 0, ey = 0, ez = 0;
         if (base == 0) {
-            LDO_LDS const int32_t* q = (LDO_LDS const int32_t*)(ep + i * (int)sizeof(Endpoint));
+            LDO_LDS const Word* q = (LDO_LDS const Word*)(ep + i * (int)sizeof(Endpoint));
             k = (uint32_t)q[0];
             es = q[1];
             ex = q[2];
@@ -1710,11 +1710,11 @@ __device__ __forceinline__ void WEng::walk_six(int d, int sg, int std_) {
 DEVNI void WEng::cb_select_and_set(int d, int prev_d) {
     bool ctcb = S->kind == LDO_MOVE_KIND_CTCB;
     // everything known of d and its neighbour, in one round of reads
-    uint4 q0 = *(LDO_LDS const uint4*)(dom.p + prev_d * 16);
+    Quad q0 = *(LDO_LDS const Quad*)(dom.p + prev_d * 16);
     int q1 = *(LDO_LDS const int8_t*)(dom.p + d * 16 + 13);
     int q2 = dident.lane(d);
     int q3 = seg.lane(d), q4 = stem.lane(d);
-    uint4 q5 = *(LDO_LDS const uint4*)(old.p + d * 16);
+    Quad q5 = *(LDO_LDS const Quad*)(old.p + d * 16);
     I3 pp = i3(uni((int32_t)q0.x), uni((int32_t)q0.y), uni((int32_t)q0.z));
     int id = uni(q2);
     if (uni(q1) != OCC_UNASSIGNED) {
@@ -1949,7 +1949,7 @@ DEVIN void WEng::cp_remove_active(int s, bool rec) {
 #ifdef __HIP_DEVICE_COMPILE__
         if (base == 0) {
             // two words tell which go; mostly none does
-            LDO_LDS const int32_t* q = (LDO_LDS const int32_t*)(ep + i * (int)sizeof(Endpoint));
+            LDO_LDS const Word* q = (LDO_LDS const Word*)(ep + i * (int)sizeof(Endpoint));
             drop = (i < n) & (q[0] == (cs | dd << 16)) & (q[1] == sg);
             if (ballot(drop) == 0) {
                 k = n < 64 ? n : 64;

@@ -42,6 +42,14 @@ LDO_HD int site_home(int x, int y, int z, int bits) {
     return (int)(h >> (32 - bits));
 }
 
+// 16 bytes of a block, and four, whatever fields lie there.  Records are written
+// field by field and read whole, or the other way round, so these accesses may
+// alias fields of any type.
+struct __attribute__((may_alias, aligned(16))) Quad {
+    uint32_t x, y, z, w;
+};
+typedef int32_t __attribute__((may_alias)) Word;
+
 // Domain record, 16 bytes.
 struct DomRec {
     int32_t x, y, z;

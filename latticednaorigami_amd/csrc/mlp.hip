@@ -221,9 +221,10 @@ __global__ void __launch_bounds__(64 * TW) mlp_tile(TileArgs g) {
         int r = i / (H / 8), c = i % (H / 8) * 8;
         uint4 v = make_uint4(0, 0, 0, 0);
         if (s0 + r < g.batch) {
-            v = *(const uint4*)(g.h1 + (size_t)(s0 + r) * H + c);
+            __builtin_memcpy(&v, __builtin_assume_aligned(g.h1 + (size_t)(s0 + r) * H + c, 16),
+                             sizeof v);
         }
-        *(uint4*)&act[0][r * TR + c] = v;
+        __builtin_memcpy(__builtin_assume_aligned(&act[0][r * TR + c], 16), &v, sizeof v);
     }
     __syncthreads();
     for (int layer = 0; layer < 2; layer++) {

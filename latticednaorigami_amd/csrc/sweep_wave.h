@@ -41,8 +41,8 @@ template <bool ALL>
 __device__ __forceinline__ void sweep_staged(const Params& P, int r, char* blk, lds_t lds,
                                              int64_t steps, const int32_t* rep_slot) {
     int n16 = (int)(P.L.stage / 16);
-    uint4* g = (uint4*)blk;
-    LDO_LDS uint4* l = (LDO_LDS uint4*)lds;
+    Quad* g = (Quad*)blk;
+    LDO_LDS Quad* l = (LDO_LDS Quad*)lds;
     int lane = threadIdx.x & 63;
     for (int i = lane; i < n16; i += 64) {
         l[i] = g[i];
@@ -57,7 +57,7 @@ template <bool ALL>
 __global__ void __launch_bounds__(64)
     ldo_sweep_lds_kernel(Params P, int64_t steps, const int32_t* rep_slot,
                          const int32_t* q_to_rep) {
-    extern __shared__ uint4 lds_block[];
+    extern __shared__ Quad lds_block[];
     if ((int)blockIdx.x >= P.n_replicas) {
         return;
     }
@@ -71,7 +71,7 @@ template <bool ALL>
 __global__ void __launch_bounds__(64)
     ldo_batch_sweep_lds_kernel(const Params* plist, const int32_t* order, int32_t n,
                                int64_t steps) {
-    extern __shared__ uint4 lds_block[];
+    extern __shared__ Quad lds_block[];
     if ((int)blockIdx.x >= n) {
         return;
     }

@@ -81,7 +81,7 @@ void sweep_one(const HostCtx& c, int r, int64_t steps, const int32_t* rep_slot) 
         return;
     }
     char* blk = c.blocks + (size_t)r * c.P.L.bytes;
-    std::vector<uint4> lds((size_t)wave_lds_bytes(c.P) / 16);
+    std::vector<Quad> lds((size_t)wave_lds_bytes(c.P) / 16);
     std::memcpy((char*)lds.data(), blk, (size_t)c.P.L.stage);
     auto sweep = wave_all_kinds(c.P) ? sweep_wave<true> : sweep_wave<false>;
     sweep(c.P, r, blk, (char*)lds.data(), steps, rep_slot);

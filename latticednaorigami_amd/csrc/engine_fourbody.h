@@ -601,8 +601,12 @@ struct FourBody {
 // Lanes of every kind run the same instructions with their results selected,
 // so a check has no branch of its own; the wavefront leaves out the junctions
 // when no lane has a candidate for one.  Positions are folded into one word
-// (x + 2^10 y + 2^20 z): every difference taken is one of chain neighbours',
-// a unit vector.  HALF: HalfTurn domains, whose twist rule is that contiguous
+// (x + 2^10 y + 2^20 z, modulo 2^32): the difference of two folded positions is
+// the folded unit vector between chain neighbours that lie side by side.  Placed
+// neighbours always do.  A trial may put a domain at a site that is not next to
+// its placed neighbour; its differences are no folded unit vectors (or look like
+// other ones, more than 1000 sites away), and its verdict and energy mean
+// nothing: the caller takes no such site, because no walk remains from it.  HALF: HalfTurn domains, whose twist rule is that contiguous
 // domains off the orientation's axis point in opposite directions.  ONE: every
 // pair has the same stacking energy, so a term's pairs are not told.
 struct FbTerm {
@@ -614,19 +618,24 @@ struct FbTerm {
 
 // a domain as a check reads it: folded position, DomRec's packed word
 struct FbWord {
-    int c;
+    uint32_t c;
     uint32_t w;
     DEV int ore() const { return (int)(w & 0xFFu); }
     DEV int partner() const { return (int)w >> 16; }
     DEV bool is_bound() const { return (w & 0xFF00u) == (uint32_t)OCC_BOUND << 8; }
 };
-DEV int fb_fold(int x, int y, int z) { return x + (y << 10) + (z << 20); }
+DEV uint32_t fb_fold(int x, int y, int z) {
+    return (uint32_t)x + ((uint32_t)y << 10) + ((uint32_t)z << 20);
+}
+// from p to q
+DEV int fb_diff(const FbWord& q, const FbWord& p) { return (int)(q.c - p.c); }
+DEV int fb_neg(int d) { return (int)(0u - (uint32_t)d); }
 // the axis of vector index o as a folded unit vector, and the vector itself
 DEV int fb_axis(int o) { return 1 << (5 * (o & 6)); }
 DEV int fb_vector(int o) { return (o & 1) ? -fb_axis(o) : fb_axis(o); }
 // index of a folded unit vector
 DEV int fb_index(int d) {
-    int m = d < 0 ? -d : d;
+    int m = d < 0 ? fb_neg(d) : d;
     return 2 * (m > 1) + 2 * (m > 1024) + (d < 0);
 }
 
@@ -672,7 +681,7 @@ struct FbChecks {
     static DEV bool stacked(int s, const FbWord& rs, int t, const FbWord& rt) {
         bool up = s < t;
         FbWord p = HALF ? rs : pick(up, rs, rt), q = HALF ? rt : pick(up, rt, rs);
-        int d = q.c - p.c, m = d < 0 ? -d : d;
+        int d = fb_diff(q, p), m = d < 0 ? fb_neg(d) : d;
         return (m != fb_axis(p.ore())) & twist_ok(p, d, q);
     }
 
@@ -699,7 +708,7 @@ struct FbChecks {
         int pb = rp.partner(), qb = rq.partner();
         bool next_to = adjacent(pb, qb);
         bool helix = next_to & (qb > pb), contig = next_to & (qb < pb);
-        int d = rq.c - rp.c, m = d < 0 ? -d : d;
+        int d = fb_diff(rq, rp), m = d < 0 ? fb_neg(d) : d;
         int po = rp.ore(), qo = rq.ore();
         bool along = m == fb_axis(po);  // the pair lies on p's axis
         bool ahead = d == fb_vector(po); // q is where p points
@@ -785,8 +794,8 @@ struct FbChecks {
             // ---- triplets (v, n, f)
             bool bk = (is_t & (back != 0)) | (is_c & (second == 0));
             int other = step(di, back);
-            int dn = rn.c - rv.c;
-            bool str = dn == rf.c - rn.c;
+            int dn = fb_diff(rn, rv);
+            bool str = dn == fb_diff(rf, rn);
             bool dcv = ((bk ? n - v : v - n) == 1) & adjacent(rv.partner(), rn.partner());
             int vb = rv.partner();
             bool on = (is_t & ((kind & (ON | CONTIG_PAIR)) == ON)) |
@@ -794,7 +803,7 @@ struct FbChecks {
             bool again = is_t & (i > 0) & ((vb == far) | (vb == f));
             bool trip = on & bv & !str & !again;
             bool off_v = dn != fb_vector(rv.ore());
-            bool off_f = rn.c - rf.c != fb_vector(rf.ore());
+            bool off_f = fb_diff(rn, rf) != fb_vector(rf.ore());
             bool may_v = fw | (is_c & (back == 0));
             bool may_f = is_c ? second == 0 : is_t & ((i == 2) | ((back != 0) & (i == 0)));
             bool both = trip & sv & sf;
@@ -841,13 +850,13 @@ struct FbChecks {
         bool flip = c1 > c2;
         FbWord lo = pick(flip, s2, s1), hi = pick(flip, s1, s2);
         jn_ok = jn_ok & stacked(j1, r1, j2, r2) & stacked(x, rx, y, ry) &
-                (hi.c - lo.c == fb_vector(lo.ore()));
+                (fb_diff(hi, lo) == fb_vector(lo.ore()));
         // directions along increasing domain index
-        int n1 = j1 < j2 ? r2.c - r1.c : r1.c - r2.c;
-        int n3 = x < y ? ry.c - rx.c : rx.c - ry.c;
+        int n1 = j1 < j2 ? fb_diff(r2, r1) : fb_diff(r1, r2);
+        int n3 = x < y ? fb_diff(ry, rx) : fb_diff(rx, ry);
         // check_junction_constraint (domain.cpp:59-67, 99-118)
         bool jv = !HALF && !twist_off_axis(lo, flip ? n3 : n1, hi);
-        int jop = n1 == n3 ? 4 : (n1 == -n3 ? 0 : 3);
+        int jop = n1 == n3 ? 4 : (n1 == fb_neg(n3) ? 0 : 3);
         out.viol = jn_ok ? (int)jv : out.viol;
         out.op = jn_ok ? (jv ? 0 : jop) : out.op;
         if (!ONE) {

@@ -562,6 +562,16 @@ int eh_get_observables(void* ctx, int32_t replica, ldo_obs* out) {
     });
 }
 
+// active endpoints that the last scaffold regrowth began with, and the LDS a
+// replica needs on the wavefront engine
+int eh_active_endpoints(void* ctx, int32_t replica) {
+    HostCtx* c = static_cast<HostCtx*>(ctx);
+    return ((const RepScalars*)(c->blocks + (size_t)replica * c->P.L.bytes))->n_active0;
+}
+int64_t eh_wave_lds_bytes(void* ctx) {
+    return wave_lds_bytes(static_cast<HostCtx*>(ctx)->P);
+}
+
 int eh_get_move_tracking(void* ctx, int32_t replica, int64_t* out, int64_t cap, int64_t* n_out) {
     HostCtx* c = static_cast<HostCtx*>(ctx);
     return guarded(c, [&]() {

@@ -2,9 +2,10 @@
 rings (segments and stacked pairs across the scaffold's ends), sequence
 specific stacking (energies that differ from pair to pair), disallowed
 misbinding, more staples than a wavefront has lanes, staples of up to eight
-domains in strides with unused slots, and centring and constraint checks every
-few steps.  Each runs step for step against the CPU oracle, on the host build
-of the engine and on the GPU, and the general engine runs beside it."""
+domains in strides with unused slots, centring and constraint checks every few
+steps, and more active endpoints than a wavefront reads at once.  Each runs step
+for step against the CPU oracle, on the host build of the engine and on the GPU,
+and the general engine runs beside it."""
 import ctypes as C
 import dataclasses
 import os
@@ -56,6 +57,32 @@ def long_staples(moves):
         flags=abi.FLAG_CTCB_SCAFFOLD_ENDPOINTS)
 
 
+def crossings(regrowth):
+    """Two rows of 200 domains joined by a staple at every column: a regrown segment
+    begins with an endpoint for each of its domains, up to 180, where a wavefront
+    reads 64 at a time and holds 64 in LDS.  Binding is weak at these temperatures,
+    so that the product of 180 weights stays a double (the oracle's has 64 bits and
+    a wider exponent)."""
+    w = 200
+    s = systems.batch_chain_system(8)
+    sites = [(i, 0, 0) for i in range(w)] + [(i, 1, 0) for i in range(w - 1, -1, -1)]
+    ores = [(0, 0, (-1) ** i) for i in range(2 * w)]
+    staples = [[i + 1, 2 * w - i] for i in range(w)]
+    chains = [systems.Chain(0, 0, sites, ores)]
+    for t, ids in enumerate(staples, start=1):
+        at = [v - 1 for v in ids]
+        chains.append(systems.Chain(t, t, [sites[i] for i in at],
+                                    [tuple(-x for x in ores[i]) for i in at]))
+    moves = [systems.Move(abi.MOVE_ORIENTATION_ROTATION, 0.1),
+             systems.Move(abi.MOVE_MET_STAPLE_EXCHANGE, 0.1),
+             systems.Move(abi.MOVE_CB_STAPLE_REGROWTH, 0.1),
+             dataclasses.replace(regrowth, freq=0.7)]
+    return dataclasses.replace(
+        s, identities=[[-(i + 1) for i in range(2 * w)]] + staples, chains=chains, moves=moves,
+        max_total_staples=w, max_type_staples=2, temps=[354.0, 358.0],
+        flags=abi.FLAG_CTCB_SCAFFOLD_ENDPOINTS)
+
+
 FORMS = {
     "ring": lambda: ring(abi.HALFTURN, systems.standard_moveset),
     "ring_three_quarter": lambda: ring(abi.THREEQUARTERTURN, systems.standard_moveset),
@@ -68,6 +95,10 @@ FORMS = {
     "crowded": crowded,
     "long_staples": lambda: long_staples(systems.standard_moveset),
     "long_staples_ctrg": lambda: long_staples(systems.ctrg_moveset),
+    "crossings": lambda: crossings(
+        systems.Move(abi.MOVE_CTCB_SCAFFOLD_REGROWTH, 1.0, 180)),
+    "crossings_ctrg": lambda: crossings(
+        systems.Move(abi.MOVE_CTRG_SCAFFOLD_REGROWTH, 1.0, 180, 1, 36)),
     "centred": lambda: raster(centering_freq=7, constraint_check_freq=11),
 }
 
@@ -75,7 +106,8 @@ FORMS = {
 def check(make, oracle_mod, name):
     s = FORMS[name]()
     print("form", name, flush=True)
-    steps = 4000 if name == "crowded" else 150 if "ctrg" in name or "jump" in name else 1500
+    slow = any(k in name for k in ("ctrg", "jump", "crossings"))
+    steps = 4000 if name == "crowded" else 150 if slow else 1500
     os.environ["LDO_SWEEP_KERNEL"] = "global"
     try:
         general = make(s, temps=s.temps)
@@ -101,6 +133,17 @@ def test_forms_on_the_host_build(host_sampler, oracle_mod, name):  # noqa: F811
     wave = check(host_sampler, oracle_mod, name)
     if name == "crowded":
         assert max(wave.observables(r)["num_staples"] for r in range(2)) > 64
+    if name.startswith("crossings"):
+        host = C.CDLL(HOST_LIB)
+        host.eh_active_endpoints.argtypes = [C.c_void_p, C.c_int32]
+        host.eh_wave_lds_bytes.argtypes = [C.c_void_p]
+        host.eh_wave_lds_bytes.restype = C.c_int64
+        assert host.eh_wave_lds_bytes(wave.h) <= 160 * 1024  # the GPU takes this engine too
+        began = set()
+        for _ in range(60):
+            wave.sweep(1)
+            began.update(host.eh_active_endpoints(wave.h, r) for r in range(2))
+        assert any(64 < n <= 128 for n in began) and max(began) > 128
 
 
 @pytest.mark.parametrize("target", ["alias", "fold"])

@@ -385,6 +385,50 @@ def case_window_temperature_swaps(sampler_cls, oracle_mod):
             x.set_windows(bad, grid, glen)
 
 
+LONG_LADDERS = {
+    "50_50_50": [50] * 3, "70_70": [70] * 2, "131": [131], "63_2_64_65": [63, 2, 64, 65]}
+
+
+def case_window_ladders_past_64_slots(sampler_cls, oracle_mod, name):
+    """Window ladders that do not fit the exchange's 64 lanes: ladders that end within a
+    set of 64 slots, pairs across its edge, more than 64 temperature-direction pairs,
+    draws numbered on from set to set, in odd and even rounds."""
+    import random
+    sizes = LONG_LADDERS[name]
+    say(f"case: four-domain system, window ladders of {sizes}, 6 rounds x 40 steps")
+    s = systems.four_domain_system(max_total_staples=8)
+    n = sum(sizes)
+    temps = [330.0 + 2.0 * k for k, size in enumerate(sizes) for _ in range(size)]
+    equal = len(sizes) > 1 and len(set(sizes)) == 1
+    if equal:
+        s.flags = abi.FLAG_WINDOW_TEMPERATURE_SWAPS
+    s.temps = temps
+    glen = 5
+    wins = [abi.Window(abi.OP_NUMFULLDOMAINS, 0, 2 + i % 3, 0, 0.0, 0.0, 1.0, 0.0, 1.0)
+            for size in sizes for i in range(size)]
+    rnd = random.Random(n)
+    grid = [rnd.uniform(-1.0, 1.0) for _ in range(n * glen)]
+    gpu = sampler_cls(s, temps=temps, exchange_mode=abi.EXCHANGE_WINDOWS)
+    ref = oracle_mod.Oracle(s, temps=temps, exchange_mode=abi.EXCHANGE_WINDOWS)
+    for x in (gpu, ref):
+        x.set_windows(wins, grid, glen)
+    for rounds in (1, 1, 2, 1, 1):
+        gpu.run(rounds, 40)
+        ref.run(rounds, 40)
+        assert gpu.permutation() == ref.permutation()
+        ag, bg = gpu.exchange_counts()
+        ar, br = ref.exchange_counts()
+        assert ag.tolist() == ar.tolist() and bg.tolist() == br.tolist()
+    for r in range(n):
+        assert_same(gpu, ref, r)
+    # swaps at every ladder, and not at every try
+    at = 0
+    for size in sizes:
+        assert size < 3 or 0 < bg[0][at:at + size].sum() < ag[0][at:at + size].sum()
+        at += size
+    assert not equal or 0 < bg[1].sum() < ag[1].sum()
+
+
 def case_mwus3d_full_size_exchanges(sampler_cls, oracle_mod):
     """The 3D umbrella workload at its full size: 64 windows x 4 temperatures
     (256 replicas of the 200-domain scaffold), exchanges every 500 steps,

@@ -201,5 +201,10 @@ def test_window_temperature_swaps(sampler_cls, oracle_mod):
     pc.case_window_temperature_swaps(sampler_cls, oracle_mod)
 
 
+@pytest.mark.parametrize("name", sorted(pc.LONG_LADDERS))
+def test_window_ladders_past_64_slots(sampler_cls, oracle_mod, name):
+    pc.case_window_ladders_past_64_slots(sampler_cls, oracle_mod, name)
+
+
 def test_exchange_and_site_eval(sampler_cls, oracle_mod):
     pc.case_exchange_and_site_eval(sampler_cls, oracle_mod)

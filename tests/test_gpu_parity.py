@@ -136,6 +136,11 @@ def test_window_temperature_swaps(sampler_cls, oracle_mod):
     pc.case_window_temperature_swaps(sampler_cls, oracle_mod)
 
 
+@pytest.mark.parametrize("name", sorted(pc.LONG_LADDERS))
+def test_window_ladders_past_64_slots(sampler_cls, oracle_mod, name):
+    pc.case_window_ladders_past_64_slots(sampler_cls, oracle_mod, name)
+
+
 def test_mwus3d_full_size_exchanges(sampler_cls, oracle_mod):
     pc.case_mwus3d_full_size_exchanges(sampler_cls, oracle_mod)
 

@@ -94,6 +94,62 @@ def test_gpu_loss_and_gradient_match_reference():
     assert np.all(np.isneginf(lp[~fin]))
 
 
+def _assert_matches(net, p, n_ident, ch, ident, legal, target):
+    """Loss, gradient and log-probabilities of one batch against the restatement.  The
+    sums agree to FP32 rounding, but where a sum lies on the boundary between two bf16
+    values the two sides round an operand of the next product apart, by 2^-8 of it at
+    most.  One such operand moves a logit by 2^-8 |h W|, 0.008 at the largest hidden
+    value (13) and weight (0.16) of these networks; the restatement's own sums in FP32
+    move 1 to 2 % of 1030 samples by more than 1e-4, the most by 0.016.  Ten such
+    operands are allowed, on one sample in twenty (two of a small batch), and four in a
+    gradient's largest entry."""
+    p = p.astype(np.float64)
+    loss, g = net.loss_grad(ch, ident, legal, target, want_grads=True)
+    ref_loss, ref_g = M.loss_grad(p, n_ident, ch, ident, legal, target)
+    assert loss == pytest.approx(ref_loss, abs=0.08)
+    L = M.layout(n_ident)
+    names = ["w1", "emb", "w1e", "b1", "w2", "b2", "w3", "b3", "w4", "b4", "total"]
+    for a, b in zip(names, names[1:]):
+        ga, gr = g[L[a]:L[b]], ref_g[L[a]:L[b]]
+        tol = 2.0 ** -6 * np.abs(gr).max()
+        assert np.abs(ga - gr).max() <= tol, (a, np.abs(ga - gr).max(), tol)
+    lp = net.log_probs(ch, ident, legal)
+    ref_lp = M.forward(p, n_ident, ch, ident, legal)["logp"]
+    fin = legal == 1
+    off = np.abs(np.where(fin, lp, 0) - np.where(fin, ref_lp, 0)).max(axis=1)
+    assert off.max() <= 0.08 and (off > 1e-4).sum() <= max(2, len(ident) // 20), np.sort(off)
+    assert np.all(np.isneginf(lp[~fin]))
+    return g
+
+
+@pytest.mark.gpu
+def test_gpu_batches_of_every_tile_remainder():
+    """One network at batch sizes around its tiles (16 samples, 32 padded columns, 4
+    samples of embedding gradient, 1024 channels), falling and rising, so that each
+    finds what larger and smaller batches left; then after set_params and after an
+    Adam step, whose packed weights have to be the new parameters'."""
+    from latticednaorigami_amd.mlp import Mlp
+    rng = np.random.default_rng(11)
+    n_ident = 5
+    p = _params(rng, n_ident).astype(np.float32)
+    net = Mlp(n_ident, max_batch=1030, params=p)
+    for n in (1030, 64, 33, 32, 17, 16, 15, 3, 1, 2, 16, 31, 33, 49, 1025):
+        print("case: MLP batch of", n, flush=True)
+        _assert_matches(net, p, n_ident, *M.random_batch(rng, n, n_ident))
+    p = _params(rng, n_ident).astype(np.float32)
+    net.set_params(p)
+    print("case: MLP after set_params", flush=True)
+    g = _assert_matches(net, p, n_ident, *M.random_batch(rng, 33, n_ident))
+    print("case: MLP after an Adam step", flush=True)
+    net.adam_step(lr=1e-2)
+    q = net.params()
+    # first step: m / c1 = g and v / c2 = g^2, up to the rounding of c1 and c2,
+    # which subtract 0.9 and 0.999 from 1 in FP32 (6e-5 of c2, half of it in the root)
+    step = p.astype(np.float64) - 1e-2 * g / (np.abs(g.astype(np.float64)) + 1e-8)
+    assert np.abs(q - step).max() < 1e-2 * 1e-4 + 1e-6
+    _assert_matches(net, q, n_ident, *M.random_batch(rng, 257, n_ident))
+
+
 @pytest.mark.gpu
 def test_gpu_training_learns_a_planted_rule():
     """Adam on ldo_mlp_loss_grad learns a rule the input decides (the target

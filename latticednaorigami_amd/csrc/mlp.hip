@@ -24,7 +24,9 @@
 // where the launches of one thing each took 440.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
+#include <cstdlib>
 #include <cstring>
 #include <random>
 #include <string>
@@ -523,6 +525,31 @@ void hcheck(hipError_t e, const char* what) {
     }
 }
 
+// Host memory that transfers go through: pinned, or ordinary memory (which the
+// runtime stages itself) where none can be had.
+struct HostBuf {
+    void* mem = nullptr;
+    bool pinned = false;
+    void alloc(size_t bytes) {
+        pinned = hipHostMalloc(&mem, bytes, hipHostMallocDefault) == hipSuccess;
+        if (!pinned) {
+            (void)hipGetLastError();
+            mem = std::malloc(bytes);
+            if (mem == nullptr) {
+                throw MlpError {LDO_E_HIP, "host memory for a batch"};
+            }
+        }
+    }
+    ~HostBuf() {
+        if (pinned) {
+            (void)hipHostFree(mem);
+        }
+        else {
+            std::free(mem);
+        }
+    }
+};
+
 struct MlpCtx {
     int n_ident = 0;
     int cap = 0;
@@ -533,10 +560,10 @@ struct MlpCtx {
     float* d_m = nullptr;
     float* d_v = nullptr;
     // one batch of samples as one transfer: channels | ident | legal | target,
-    // each part at a multiple of 16 bytes (upload_batch), and the same in
-    // pinned host memory
+    // each part at a multiple of 16 bytes (upload_batch), and the same on the
+    // host
     uint8_t* d_in = nullptr;
-    uint8_t* h_in = nullptr;
+    HostBuf h_in;
     size_t in_bytes = 0;
     uint8_t* d_ch = nullptr;
     int32_t* d_id = nullptr;
@@ -547,7 +574,7 @@ struct MlpCtx {
     unsigned short* tr = nullptr; // transposed operands of the weight gradients
     float *dz1 = nullptr, *dz2 = nullptr, *dz3 = nullptr, *dz4 = nullptr, *logp = nullptr;
     double* d_loss = nullptr;
-    void* h_out = nullptr; // pinned: losses or log-probabilities
+    HostBuf h_out; // losses or log-probabilities
     hipStream_t stream = nullptr;
     std::string err;
 };
@@ -584,11 +611,6 @@ void free_mlp(MlpCtx* c) {
     for (void* p: ptrs) {
         if (p) {
             (void)hipFree(p);
-        }
-    }
-    for (void* p: {(void*)c->h_in, c->h_out}) {
-        if (p) {
-            (void)hipHostFree(p);
         }
     }
     if (c->stream) {
@@ -645,17 +667,18 @@ void upload_batch(MlpCtx& c, int batch, const uint8_t* ch, const int32_t* id, co
     // are free here
     size_t o_id = part_bytes((size_t)batch * NS), o_lg = o_id + part_bytes((size_t)batch * 4),
            o_tg = o_lg + part_bytes((size_t)batch * NO), n = o_tg + (size_t)batch * 4;
-    std::memcpy(c.h_in, ch, (size_t)batch * NS);
-    std::memcpy(c.h_in + o_id, id, (size_t)batch * 4);
-    std::memcpy(c.h_in + o_lg, legal, (size_t)batch * NO);
+    uint8_t* h = (uint8_t*)c.h_in.mem;
+    std::memcpy(h, ch, (size_t)batch * NS);
+    std::memcpy(h + o_id, id, (size_t)batch * 4);
+    std::memcpy(h + o_lg, legal, (size_t)batch * NO);
     if (tgt) {
-        std::memcpy(c.h_in + o_tg, tgt, (size_t)batch * 4);
+        std::memcpy(h + o_tg, tgt, (size_t)batch * 4);
     }
     c.d_ch = c.d_in;
     c.d_id = (int32_t*)(c.d_in + o_id);
     c.d_legal = c.d_in + o_lg;
     c.d_tgt = (int32_t*)(c.d_in + o_tg);
-    hcheck(hipMemcpyAsync(c.d_in, c.h_in, n, hipMemcpyHostToDevice, c.stream), "copy batch");
+    hcheck(hipMemcpyAsync(c.d_in, h, n, hipMemcpyHostToDevice, c.stream), "copy batch");
 }
 
 // the transposed operands of a batch: h1, h2, h3, dz2, dz3 ([H][cols]), dz4 ([NP][cols])
@@ -715,9 +738,8 @@ int ldo_mlp_create(int32_t n_ident, int32_t max_batch, const float* params, uint
         c->in_bytes = part_bytes((size_t)max_batch * NS) + 2 * part_bytes((size_t)max_batch * 4) +
                       part_bytes(bo);
         dalloc(c->d_in, c->in_bytes, "batch");
-        hcheck(hipHostMalloc((void**)&c->h_in, c->in_bytes), "pinned batch");
-        hcheck(hipHostMalloc(&c->h_out, std::max(bo * sizeof(float), max_batch * sizeof(double))),
-               "pinned results");
+        c->h_in.alloc(c->in_bytes);
+        c->h_out.alloc(std::max(bo * sizeof(float), max_batch * sizeof(double)));
         dalloc(c->d_pk, PK_TOTAL, "packed weights");
         dalloc(c->h1, bh, "activations");
         dalloc(c->tr, (5 * H + NP) * cols, "transposed operands");
@@ -811,7 +833,7 @@ int ldo_mlp_loss_grad(void* mlp, int32_t batch, const uint8_t* channels, const i
         upload_batch(*c, batch, channels, ident, legal, target);
         network(*c, batch, true);
         hcheck(hipGetLastError(), "loss/grad kernels");
-        double* l = (double*)c->h_out;
+        double* l = (double*)c->h_out.mem;
         hcheck(hipMemcpyAsync(l, c->d_loss, batch * sizeof(double), hipMemcpyDeviceToHost,
                               c->stream),
                "download loss");
@@ -854,10 +876,10 @@ int ldo_mlp_log_probs(void* mlp, int32_t batch, const uint8_t* channels, const i
         network(*c, batch, false);
         hcheck(hipGetLastError(), "forward kernels");
         size_t bytes = (size_t)batch * NO * sizeof(float);
-        hcheck(hipMemcpyAsync(c->h_out, c->logp, bytes, hipMemcpyDeviceToHost, c->stream),
+        hcheck(hipMemcpyAsync(c->h_out.mem, c->logp, bytes, hipMemcpyDeviceToHost, c->stream),
                "download log-probs");
         hcheck(hipStreamSynchronize(c->stream), "forward sync");
-        std::memcpy(out, c->h_out, bytes);
+        std::memcpy(out, c->h_out.mem, bytes);
     });
 }
 

@@ -2,6 +2,7 @@
 pinned by finite differences, and the HIP training kernels checked against
 it on an MI355X."""
 import os
+import subprocess
 import sys
 
 import numpy as np
@@ -148,6 +149,55 @@ def test_gpu_batches_of_every_tile_remainder():
     step = p.astype(np.float64) - 1e-2 * g / (np.abs(g.astype(np.float64)) + 1e-8)
     assert np.abs(q - step).max() < 1e-2 * 1e-4 + 1e-6
     _assert_matches(net, q, n_ident, *M.random_batch(rng, 257, n_ident))
+
+
+NO_PINNED = r"""
+#include <stddef.h>
+static int asked;
+/* hipErrorOutOfMemory, as where no pinned memory is left */
+int hipHostMalloc(void** p, size_t n, unsigned flags) { *p = 0; asked++; return 2; }
+int pinned_asked(void) { return asked; }
+"""
+
+# scores a batch and takes a training step; with a shim as argument, behind it
+SCORE = r"""
+import ctypes as C, hashlib, sys
+import numpy as np
+shim = C.CDLL(sys.argv[1], C.RTLD_GLOBAL) if len(sys.argv) > 1 else None
+import mlp_ref as M
+from latticednaorigami_amd import systems
+from latticednaorigami_amd.mlp import Mlp
+from latticednaorigami_amd.sampler import Sampler
+rng = np.random.default_rng(3)
+net = Mlp(5, max_batch=40, seed=9)
+asked = shim.pinned_asked() if shim else 2
+ch, ident, legal, target = M.random_batch(rng, 33, 5)
+loss, g = net.loss_grad(ch, ident, legal, target, want_grads=True)
+lp = net.log_probs(ch, ident, legal)
+net.adam_step()
+net.close()
+s = Sampler(systems.four_domain_system(), temps=[330.0])
+s.sweep(200)
+d = hashlib.sha256(lp.tobytes() + np.float64(loss).tobytes()).hexdigest()
+print(asked, d, s.observables(0)["energy"], len(s.config(0)))
+"""
+
+
+@pytest.mark.gpu
+def test_gpu_network_without_pinned_memory(tmp_path):
+    """Where the runtime has no pinned memory to give, a network (and a sampler) works
+    through ordinary memory, with the same results."""
+    print("case: MLP and sampler without pinned memory", flush=True)
+    src = tmp_path / "no_pinned.c"
+    src.write_text(NO_PINNED)
+    shim = tmp_path / "no_pinned.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(shim), str(src)], check=True)
+    env = dict(os.environ, PYTHONPATH=os.pathsep.join([ROOT, os.path.join(ROOT, "oracle")]))
+    out = [subprocess.run([sys.executable, "-c", SCORE, *args], env=env, check=True, timeout=100,
+                          capture_output=True, text=True).stdout.split()
+           for args in ([], [str(shim)])]
+    assert int(out[1][0]) >= 2  # the shim was asked for the network's two buffers
+    assert out[0][1:] == out[1][1:]
 
 
 @pytest.mark.gpu

@@ -1542,11 +1542,12 @@ void group_batch(BatchCtx& b) {
     bupload(b, b.d_order, order, "copy order");
 }
 
-// Launches `steps` steps on every chain with the batch's sweep kernel and
-// returns the kernel time.
-double batch_launch(BatchCtx& b, int kernel, int64_t steps) {
-    hip_check(hipEventRecord(b.ev0, b.stream), "event record");
-    if (kernel == LDO_BATCH_LDS) {
+// The LDS sweep's groups side by side, forked from and joined to the batch's
+// stream.  Where a call fails on the way, groups launched before it are running
+// on their chains and the batch's stream does not wait for them: they are
+// waited for here, before the error is told.
+void launch_groups(BatchCtx& b, int64_t steps) {
+    try {
         for (size_t g = 0; g < b.groups.size(); g++) {
             hipStream_t st = g == 0 ? b.stream : b.side[g - 1];
             if (g > 0) {
@@ -1562,6 +1563,20 @@ double batch_launch(BatchCtx& b, int kernel, int64_t steps) {
         for (hipEvent_t e: b.side_ev) {
             hip_check(hipStreamWaitEvent(b.stream, e, 0), "join");
         }
+    } catch (...) {
+        for (hipStream_t st: b.side) {
+            (void)hipStreamSynchronize(st);
+        }
+        throw;
+    }
+}
+
+// Launches `steps` steps on every chain with the batch's sweep kernel and
+// returns the kernel time.
+double batch_launch(BatchCtx& b, int kernel, int64_t steps) {
+    hip_check(hipEventRecord(b.ev0, b.stream), "event record");
+    if (kernel == LDO_BATCH_LDS) {
+        launch_groups(b, steps);
     }
     else if (kernel == LDO_BATCH_WAVE || kernel == LDO_BATCH_WAVE_SOLO) {
         hipLaunchKernelGGL(ldo_batch_sweep_kernel, dim3(b.n), dim3(64), 0, b.stream, b.d_params,

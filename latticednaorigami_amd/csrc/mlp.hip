@@ -581,20 +581,26 @@ struct MlpCtx {
 
 std::string g_mlp_create_error;
 
+// Runs f; after an error nothing of the call stays on its way to or from the
+// caller's memory and the batch's.
 template <class F>
 int mguarded(MlpCtx* c, F f) {
     std::string& err = c ? c->err : g_mlp_create_error;
+    int code = LDO_E_HIP;
     try {
         f();
         err.clear();
         return LDO_OK;
     } catch (MlpError& e) {
         err = e.msg;
-        return e.code;
+        code = e.code;
     } catch (std::exception& e) {
         err = e.what();
-        return LDO_E_HIP;
     }
+    if (c && c->stream) {
+        (void)hipStreamSynchronize(c->stream);
+    }
+    return code;
 }
 
 template <class T>
@@ -663,8 +669,8 @@ void upload_batch(MlpCtx& c, int batch, const uint8_t* ch, const int32_t* id, co
             throw MlpError {LDO_E_ARG, "target is not a legal output"};
         }
     }
-    // every call that reads these buffers ends with its stream idle, so they
-    // are free here
+    // every call that reads these buffers ends with its stream idle, after an
+    // error too (mguarded), so they are free here
     size_t o_id = part_bytes((size_t)batch * NS), o_lg = o_id + part_bytes((size_t)batch * 4),
            o_tg = o_lg + part_bytes((size_t)batch * NO), n = o_tg + (size_t)batch * 4;
     uint8_t* h = (uint8_t*)c.h_in.mem;

@@ -318,9 +318,9 @@ extern "C" __global__ void __launch_bounds__(64)
         __syncthreads();
     }
 #endif
-    const int32_t* src = (const int32_t*)P.blocks;
+    const Word* src = (const Word*)P.blocks;
     for (int i = threadIdx.x; i < (int)(sizeof(RepScalars) / 4); i += 64) {
-        ((int32_t*)(out + k))[i] = src[i];
+        ((Word*)(out + k))[i] = src[i];
     }
 }
 
